@@ -24,22 +24,19 @@
 
 namespace fwix {
 
-template <int N>
-struct BRowCfg {
-  static constexpr int NB = row_nb(N);
-  static constexpr int V = NB * N / 64;
-  static constexpr int LDSW = NB * padded(N);
-};
-
+// row iy of model plane im of the edge-padded slowness slice, and its node ix
+__device__ __forceinline__ const float2* slow_row(const KArgs& a, int im, int iy) {
+  return a.slow + (size_t)(im * a.ny + (iy < a.ny ? iy : a.ny - 1)) * a.nx;
+}
+__device__ __forceinline__ float2 slow_at(const KArgs& a, const float2* row, int ix) {
+  return row[ix < a.nx ? ix : a.nx - 1];
+}
 // c_it * s~^(-1/2-it), s~ = Re s + i (Im s - eps_s Re s), from the edge-padded
 // slowness slice (propagator/src/scatter.cu:61-106, pad_fwd :240-277,
 // Taylor coefficients Scatter.h:73).  s^(-1/2) is the reciprocal of the
 // principal square root, identical to |s|^(-1/2) e^{-i arg(s)/2}
 // (scatter.cu:6-21); higher terms multiply by 1/s.
-__device__ __forceinline__ void scatter_factors(const KArgs& a, int im, int iy, int ix, float2& rsq, float2& inv) {
-  const int yy = iy < a.ny ? iy : a.ny - 1;
-  const int xx = ix < a.nx ? ix : a.nx - 1;
-  const float2 s = a.slow[(unsigned)((im * a.ny + yy) * a.nx + xx)];
+__device__ __forceinline__ void scatter_factors(const KArgs& a, float2 s, float2& rsq, float2& inv) {
   const float sr = s.x, si = s.y - a.eps_s * s.x;
   // principal sqrt q of (sr, si), from the hardware square root and
   // reciprocal (1 ulp each); |q|^2 = |s~| = r gives both factors from 1/r
@@ -59,10 +56,7 @@ __device__ __forceinline__ void scatter_factors(const KArgs& a, int im, int iy, 
   inv = make_float2(sr * is2, -si * is2);              // 1/s~ = conj(s~)/|s~|^2
 }
 // the same factors in float64 arithmetic (from the complex64 slowness)
-__device__ __forceinline__ void scatter_factors(const KArgs& a, int im, int iy, int ix, double2& rsq, double2& inv) {
-  const int yy = iy < a.ny ? iy : a.ny - 1;
-  const int xx = ix < a.nx ? ix : a.nx - 1;
-  const float2 s = a.slow[(unsigned)((im * a.ny + yy) * a.nx + xx)];
+__device__ __forceinline__ void scatter_factors(const KArgs& a, float2 s, double2& rsq, double2& inv) {
   const double sr = s.x, si = (double)s.y - (double)a.eps_s * s.x;
   const double r = sqrt(fma(sr, sr, si * si));
   double qr, qi;
@@ -79,59 +73,50 @@ __device__ __forceinline__ void scatter_factors(const KArgs& a, int im, int iy, 
   const double is2 = ir * ir;
   inv = make_double2(sr * is2, -si * is2);
 }
-// taper weight of node (i, row j) in the arithmetic type T
-__device__ __forceinline__ float tap_of(const KArgs& a, int i, int j, float2*) { return a.tapx[i] * a.tapy[j]; }
-__device__ __forceinline__ double tap_of(const KArgs& a, int i, int j, double2*) { return a.tapx64[i] * a.tapy64[j]; }
+// taper weights of the row and the column axis in the arithmetic type T
+__device__ __forceinline__ const float* tapx_of(const KArgs& a, float2*) { return a.tapx; }
+__device__ __forceinline__ const double* tapx_of(const KArgs& a, double2*) { return a.tapx64; }
+__device__ __forceinline__ const float* tapy_of(const KArgs& a, float2*) { return a.tapy; }
+__device__ __forceinline__ const double* tapy_of(const KArgs& a, double2*) { return a.tapy64; }
 
 __device__ __forceinline__ float taylor_coef(int it) {  // Scatter.h:73
   return it == 0 ? 1.f : it == 1 ? 0.5f : it == 2 ? 0.375f : it == 3 ? 0.3125f : 0.2734375f;
 }
 
+// whether any row of this wave lies in the model region (y < ny)
+template <int N, class T>
+__device__ __forceinline__ bool wave_in_model(const KArgs& a, const RowLane<N, T>& w) {
+  return __any(w.live && w.iy < a.ny);
+}
+
 // K = scale * F_x( U * ds ) on the model region (x < nx, y < ny), zero elsewhere
 template <int N, bool MAP>
-__global__ __launch_bounds__(kThreads) void k_rows_ic_fwd(KArgs a) {
-  using C = BRowCfg<N>;
-  using F = WaveFft<N, C::NB, false, false, PadLds<N>>;
-  __shared__ float2 lds[kWaves * C::LDSW];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nrows = a.np * a.NY;
-  const int rb = (blockIdx.x * kWaves + wave) * C::NB;
-  // twiddles in LDS: a global twiddle load would wait (one counter for all
-  // vector memory operations) for every load still in flight
-  __shared__ float2 twl[N];
-  for (int i = threadIdx.x; i < N; i += kThreads) twl[i] = a.twx[i];
-  __syncthreads();
-  if (rb >= nrows) return;
+__global__ __launch_bounds__(kRowThreads) void k_rows_ic_fwd(KArgs a) {
+  using F = LaneFft<N>;
+  __shared__ float2 lds[kRowWaves * F::NB * F::STRIDE];
+  __shared__ float2 twl[F::TW];
+  const RowLane<N, float2> w(a);
+  float2* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   // rows of the padding (y >= ny) carry no product: their spectrum is zero
-  bool any = false;
-  for (int b = 0; b < C::NB; ++b) {
-    const int lr = rb + b;
-    if (lr < nrows && lr % a.NY < a.ny) any = true;
-  }
-  float2 v[C::V];
+  const bool any = wave_in_model<N>(a, w);
+  float2 v[F::V];
 #pragma unroll
-  for (int e = 0; e < C::V; ++e) {
-    int b, i;
-    edge_pos<N, C::NB, F::P::first(), false>(lane, e, b, i);
-    const int lr = rb + b;
-    v[e] = czero();
-    if (lr < nrows) {
-      const int p = lr / a.NY, iy = lr - p * a.NY;
-      if (iy < a.ny && i < a.nx) {
-        const float2 u = a.bg[(unsigned)(lr * N + i)];
-        const float2 m = a.dslow[(unsigned)((model_iw<MAP>(a, plane_iw(a, p)) * a.ny + iy) * a.nx + i)];
-        v[e] = cmul(u, m);
-      }
-    }
+  for (int e = 0; e < F::V; ++e) v[e] = czero();
+  if (any) {
+    const RowBuf<N, float2> bg(a.bg, w, false);
+    const float2* ds = a.dslow + (size_t)(model_iw<MAP>(a, w.iw) * a.ny + (w.iy < a.ny ? w.iy : 0)) * a.nx;
+    const int nx = w.live && w.iy < a.ny ? a.nx : 0;
+    in_groups<F>(v, a.nx, [&](int e) {
+      const int i = w.l + F::first_c(e);
+      return cmul(bg.load_if(i < nx, F::first_c(e)), ds[i < nx ? i : 0]);
+    });
   }
-  if (any) F::run(v, lds + wave * C::LDSW, twl, lane);
+  row_twiddles<N>(twl, a.twx);
+  __syncthreads();
+  if (any) F::template run<false>(v, line, twl, w.l);
+  const RowBuf<N, float2> K(a.K, w, a.quad != 0);
 #pragma unroll
-  for (int e = 0; e < C::V; ++e) {
-    int b, i;
-    edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-    const int lr = rb + b;
-    if (lr < nrows) a.K[widx(a, lr, i, N)] = cscale(v[e], a.scale);
-  }
+  for (int e = 0; e < F::V; ++e) K.store(cscale(v[e], a.scale), F::last_c(e));
 }
 
 // Sum of the Taylor terms in space:
@@ -147,148 +132,97 @@ __global__ __launch_bounds__(kThreads) void k_rows_ic_fwd(KArgs a) {
 // general form holds the running sum and two factor arrays across every
 // transform).
 template <int N, bool BORN, bool MAP, class T = float2, bool ONE = false>
-__global__ __launch_bounds__(kThreads) void k_rows_scatter(KArgs a) {
-  using C = BRowCfg<N>;
+__global__ __launch_bounds__(kRowThreads) void k_rows_scatter(KArgs a) {
+  using F = LaneFft<N, T>;
   using S = real_of<T>;
-  using Fi = WaveFft<N, C::NB, false, true, PadLds<N>, T>;
-  using F = WaveFft<N, C::NB, false, false, PadLds<N>, T>;
-  __shared__ T lds[kWaves * C::LDSW];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nrows = a.np * a.NY;
-  const int rb = (blockIdx.x * kWaves + wave) * C::NB;
-  // twiddles in LDS: inside the term loops a global load would wait (one
-  // counter for all vector memory operations) for the term stores / the next
-  // term's loads still in flight
-  __shared__ T twl[N];
-  const T* twg = twx_of(a, (T*)nullptr);
-  for (int i = threadIdx.x; i < N; i += kThreads) twl[i] = twg[i];
-  __syncthreads();
-  if (rb >= nrows) return;
-  T* wl = lds + wave * C::LDSW;
-  // scattering source v of node (lr, i): U_z * ds_z on the model region
+  __shared__ T lds[kRowWaves * F::NB * F::STRIDE];
+  __shared__ T twl[F::TW];
+  const RowLane<N, T> w(a);
+  T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
+  const int im = model_iw<MAP>(a, w.iw);
+  const float2* slow = slow_row(a, im, w.iy);
+  // scattering source v at column l + C: U_z * ds_z on the model region
   // (BORN) or the input row
-  auto source = [&](int lr, int p, int iy, int i) -> T {
+  const RowBuf<N, T> src(BORN ? a.bg : a.in, w, false);
+  const float2* ds = BORN ? a.dslow + (size_t)(im * a.ny + (w.iy < a.ny ? w.iy : 0)) * a.nx : nullptr;
+  const int nx = w.live && w.iy < a.ny ? a.nx : 0;
+  auto source = [&](int C) -> T {
     if constexpr (BORN) {
-      if (iy < a.ny && i < a.nx)
-        return cmul(from_f2<T>(a.bg[(unsigned)(lr * N + i)]),
-                    from_f2<T>(a.dslow[(unsigned)((model_iw<MAP>(a, plane_iw(a, p)) * a.ny + iy) * a.nx + i)]));
-      return cz<T>();
+      const int i = w.l + C;
+      return cmul(from_f2<T>(src.load_if(i < nx, C)), from_f2<T>(ds[i < nx ? i : 0]));
     } else {
-      return from_f2<T>(a.in[(unsigned)(lr * N + i)]);
+      return from_f2<T>(src.load(C));
     }
   };
-  T acc[C::V];
+  // the sum y of node e times -i w dz / 2 (propagator/src/scatter.cu:155-195),
+  // and for BORN with the wavefield added and tapered
+  const S h = (S)(0.5f * a.w[w.iw] * a.dz);
+  const RowBuf<N, T> addin(BORN ? a.addin : a.in, w, false);
+  const S ty = BORN ? tapy_of(a, (T*)nullptr)[w.iy] : (S)1;
+  const S* tx = BORN ? tapx_of(a, (T*)nullptr) + w.l : nullptr;
+  auto finish = [&](int e, T y) -> T {
+    y = CX<T>::mk(h * y.y, -h * y.x);
+    if constexpr (BORN) {
+      y = cadd(y, from_f2<T>(addin.load(F::first_c(e))));
+      y = cscale(y, tx[F::first_c(e)] * ty);
+    }
+    return y;
+  };
+  T acc[F::V];
   if constexpr (ONE) {
+    const RowBuf<N, T> W(a.W, w, a.quad != 0);
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, Fi::P::first(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      acc[e] = lr < nrows ? from_f2<T>(a.W[widx(a, lr, i, N)]) : cz<T>();
-    }
-    Fi::run(acc, wl, twl, lane);
+    for (int e = 0; e < F::V; ++e) acc[e] = from_f2<T>(W.load(F::last_c(e)));
+  }
+  row_twiddles<N>(twl, twx_of(a, (T*)nullptr));
+  __syncthreads();
+  if (w.empty()) return;
+  if constexpr (ONE) {
+    F::template run<true>(acc, line, twl, w.l);
     const S c = (S)taylor_coef(1) * (S)a.scale;  // the inverse row transform's 1/sqrt(NX)
-    // the lane index made opaque here: the per-element offsets are formed
-    // after the transform instead of held in registers across it
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, Fi::P::last(), false>(ln, e, b, i);
-      const int lr = rb + b;
-      if (lr < nrows) {
-        const int p = lr / a.NY, iy = lr - p * a.NY;
-        T pw, inv;
-        scatter_factors(a, model_iw<MAP>(a, plane_iw(a, p)), iy, i, pw, inv);
-        const T v = source(lr, p, iy, i);
-        const T pw1 = cmul(pw, inv);
-        acc[e] = cadd(cmul(v, pw), cscale(cmul(acc[e], pw1), c));  // c_0 = 1
-      } else {
-        acc[e] = cz<T>();
-      }
-    }
+    in_groups<F>(acc, N, [&](int e) {
+      T pw, inv;
+      scatter_factors(a, slow_at(a, slow, w.l + F::first_c(e)), pw, inv);
+      const T v = source(F::first_c(e));
+      const T pw1 = cmul(pw, inv);
+      return finish(e, cadd(cmul(v, pw), cscale(cmul(acc[e], pw1), c)));  // c_0 = 1
+    });
   } else {
-    T pw[C::V], inv[C::V];
+    T pw[F::V], inv[F::V];
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, Fi::P::last(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      acc[e] = cz<T>();
-      pw[e] = cz<T>();
-      inv[e] = cz<T>();
-      if (lr < nrows) {
-        const int p = lr / a.NY, iy = lr - p * a.NY;
-        scatter_factors(a, model_iw<MAP>(a, plane_iw(a, p)), iy, i, pw[e], inv[e]);
-        acc[e] = cmul(source(lr, p, iy, i), pw[e]);  // c_0 = 1
-        pw[e] = cmul(pw[e], inv[e]);
-      }
+    for (int e = 0; e < F::V; ++e) {
+      scatter_factors(a, slow_at(a, slow, w.l + F::first_c(e)), pw[e], inv[e]);
+      acc[e] = cmul(source(F::first_c(e)), pw[e]);  // c_0 = 1
+      pw[e] = cmul(pw[e], inv[e]);
     }
     for (int it = 1; it < a.nterm; ++it) {
-      const float2* W = a.W + (size_t)(it - 1) * a.wstride;
-      T x[C::V];
+      const RowBuf<N, T> W(a.W + (size_t)(it - 1) * a.wstride, w, a.quad != 0);
+      T x[F::V];
 #pragma unroll
-      for (int e = 0; e < C::V; ++e) {
-        int b, i;
-        edge_pos<N, C::NB, Fi::P::first(), false>(lane, e, b, i);
-        const int lr = rb + b;
-        x[e] = lr < nrows ? from_f2<T>(W[widx(a, lr, i, N)]) : cz<T>();
-      }
-      Fi::run(x, wl, twl, lane);
+      for (int e = 0; e < F::V; ++e) x[e] = from_f2<T>(W.load(F::last_c(e)));
+      F::template run<true>(x, line, twl, w.l);
       const S c = (S)taylor_coef(it) * (S)a.scale;  // the inverse row transform's 1/sqrt(NX)
 #pragma unroll
-      for (int e = 0; e < C::V; ++e) {
+      for (int e = 0; e < F::V; ++e) {
         acc[e] = cadd(acc[e], cscale(cmul(x[e], pw[e]), c));   // c_it s~^(-1/2-it) * term
         pw[e] = cmul(pw[e], inv[e]);
       }
     }
-  }
-  // acc *= -i * (w dz / 2)     (propagator/src/scatter.cu:155-195)
-#pragma unroll
-  for (int e = 0; e < C::V; ++e) {
-    int b, i;
-    edge_pos<N, C::NB, Fi::P::last(), false>(lane, e, b, i);
-    const int lr = rb + b;
-    if (lr < nrows) {
-      const int p = lr / a.NY;
-      const S h = (S)(0.5f * a.w[plane_iw(a, p)] * a.dz);
-      acc[e] = CX<T>::mk(h * acc[e].y, -h * acc[e].x);
-    }
+    in_groups<F>(acc, N, [&](int e) { return finish(e, acc[e]); });
   }
   if constexpr (!BORN) {
+    const RowBuf<N, T> out(a.out, w, false);
+    if (a.add) {
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, Fi::P::last(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      if (lr < nrows) {
-        const unsigned idx = lr * N + i;
-        T y = acc[e];
-        if (a.add) y = cadd(y, from_f2<T>(a.out[idx]));
-        a.out[idx] = to_f2(y);
-      }
+      for (int e = 0; e < F::V; ++e) acc[e] = cadd(acc[e], from_f2<T>(out.load(F::first_c(e))));
     }
+#pragma unroll
+    for (int e = 0; e < F::V; ++e) out.store(to_f2(acc[e]), F::first_c(e));
   } else {
-    static_assert(Fi::P::last() == F::P::first(), "register hand-off needs mirrored plans");
+    F::template run<false>(acc, line, twl, w.l);
+    const RowBuf<N, T> K(a.K, w, a.quad != 0);
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::first(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      if (lr < nrows) {
-        T y = cadd(acc[e], from_f2<T>(a.addin[(unsigned)(lr * N + i)]));
-        acc[e] = cscale(y, tap_of(a, i, lr % a.NY, (T*)nullptr));
-      }
-    }
-    F::run(acc, wl, twl, lane);
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      if (lr < nrows) a.K[widx(a, lr, i, N)] = to_f2(cscale(acc[e], a.scale));
-    }
+    for (int e = 0; e < F::V; ++e) K.store(to_f2(cscale(acc[e], (S)a.scale)), F::last_c(e));
   }
 }
 
@@ -300,116 +234,69 @@ __global__ __launch_bounds__(kThreads) void k_rows_scatter(KArgs a) {
 // ONE: the launch has exactly one Taylor order (nterm == 2), a separate
 // instantiation so that the general form's per-order factors cost it no registers.
 template <int N, bool FUSED, bool MAP, class T = float2, bool ONE = false>
-__global__ __launch_bounds__(kThreads) void k_rows_scatter_adj(KArgs a) {
-  using C = BRowCfg<N>;
+__global__ __launch_bounds__(kRowThreads) void k_rows_scatter_adj(KArgs a) {
+  using F = LaneFft<N, T>;
   using S = real_of<T>;
-  using F = WaveFft<N, C::NB, false, false, PadLds<N>, T>;
-  using Fi = WaveFft<N, C::NB, false, true, PadLds<N>, T>;
-  static_assert(Fi::P::last() == F::P::first(), "register hand-off needs mirrored plans");
-  __shared__ T lds[kWaves * C::LDSW];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nrows = a.np * a.NY;
-  const int rb = (blockIdx.x * kWaves + wave) * C::NB;
-  // twiddles in LDS: inside the term loops a global load would wait (one
-  // counter for all vector memory operations) for the term stores / the next
-  // term's loads still in flight
-  __shared__ T twl[N];
-  const T* twg = twx_of(a, (T*)nullptr);
-  for (int i = threadIdx.x; i < N; i += kThreads) twl[i] = twg[i];
+  __shared__ T lds[kRowWaves * F::NB * F::STRIDE];
+  __shared__ T twl[F::TW];
+  const RowLane<N, T> w(a);
+  T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
+  T u[F::V];
+  {
+    const RowBuf<N, T> in(FUSED ? a.K : a.in, w, FUSED && a.quad != 0);
+#pragma unroll
+    for (int e = 0; e < F::V; ++e) u[e] = from_f2<T>(in.load(FUSED ? F::last_c(e) : F::first_c(e)));
+  }
+  row_twiddles<N>(twl, twx_of(a, (T*)nullptr));
   __syncthreads();
-  if (rb >= nrows) return;
-  T* wl = lds + wave * C::LDSW;
-  T u[C::V];
+  if (w.empty()) return;
   if constexpr (FUSED) {
+    F::template run<true>(u, line, twl, w.l);
+    const RowBuf<N, T> out(a.out, w, false);
+    const S ty = tapy_of(a, (T*)nullptr)[w.iy];
+    const S* tx = tapx_of(a, (T*)nullptr) + w.l;
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, Fi::P::first(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      u[e] = lr < nrows ? from_f2<T>(a.K[widx(a, lr, i, N)]) : cz<T>();
-    }
-    Fi::run(u, wl, twl, lane);
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, Fi::P::last(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      if (lr < nrows) {
-        u[e] = cscale(u[e], (S)a.scale * tap_of(a, i, lr % a.NY, (T*)nullptr));
-        a.out[(unsigned)(lr * N + i)] = to_f2(u[e]);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::first(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      u[e] = lr < nrows ? from_f2<T>(a.in[(unsigned)(lr * N + i)]) : cz<T>();
+    for (int e = 0; e < F::V; ++e) {
+      u[e] = cscale(u[e], (S)a.scale * (tx[F::first_c(e)] * ty));
+      out.store(to_f2(u[e]), F::first_c(e));
     }
   }
   if (a.nterm < 2) return;
+  const float2* slow = slow_row(a, model_iw<MAP>(a, w.iw), w.iy);
+  const S h = (S)(0.5f * a.w[w.iw] * a.dz);   // scatter.cu:197-238
   if constexpr (ONE) {  // one Taylor order: x = conj(c_1 s~^(-3/2)) * u, nothing carried to a next order
     const S c = (S)taylor_coef(1);
+    in_groups<F>(u, N, [&](int e) {
+      const T v = CX<T>::mk(-h * u[e].y, h * u[e].x);
+      T rsq, inv;
+      scatter_factors(a, slow_at(a, slow, w.l + F::first_c(e)), rsq, inv);
+      return cscale(cmulc(v, cmul(rsq, inv)), c);
+    });
+    F::template run<false>(u, line, twl, w.l);
+    const RowBuf<N, T> W(a.W, w, a.quad != 0);
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::first(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      T x = cz<T>();
-      if (lr < nrows) {
-        const int p = lr / a.NY;
-        const S h = (S)(0.5f * a.w[plane_iw(a, p)] * a.dz);   // scatter.cu:197-238
-        const T v = CX<T>::mk(-h * u[e].y, h * u[e].x);
-        T rsq, inv;
-        scatter_factors(a, model_iw<MAP>(a, plane_iw(a, p)), lr - p * a.NY, i, rsq, inv);
-        x = cscale(cmulc(v, cmul(rsq, inv)), c);
-      }
-      u[e] = x;
-    }
-    F::run(u, wl, twl, lane);
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      if (lr < nrows) a.W[widx(a, lr, i, N)] = to_f2(cscale(u[e], a.scale));
-    }
+    for (int e = 0; e < F::V; ++e) W.store(to_f2(cscale(u[e], (S)a.scale)), F::last_c(e));
     return;
   } else {
-    T pw[C::V], inv[C::V];
+    T pw[F::V], inv[F::V];
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::first(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      pw[e] = cz<T>();
-      inv[e] = cz<T>();
-      if (lr < nrows) {
-        const int p = lr / a.NY;
-        const S h = (S)(0.5f * a.w[plane_iw(a, p)] * a.dz);   // scatter.cu:197-238
-        u[e] = CX<T>::mk(-h * u[e].y, h * u[e].x);
-        scatter_factors(a, model_iw<MAP>(a, plane_iw(a, p)), lr - p * a.NY, i, pw[e], inv[e]);
-        pw[e] = cmul(pw[e], inv[e]);                          // start at order 1
-      }
+    for (int e = 0; e < F::V; ++e) {
+      u[e] = CX<T>::mk(-h * u[e].y, h * u[e].x);
+      scatter_factors(a, slow_at(a, slow, w.l + F::first_c(e)), pw[e], inv[e]);
+      pw[e] = cmul(pw[e], inv[e]);                          // start at order 1
     }
     for (int it = 1; it < a.nterm; ++it) {
-      T x[C::V];
+      T x[F::V];
       const S c = (S)taylor_coef(it);
 #pragma unroll
-      for (int e = 0; e < C::V; ++e) {
+      for (int e = 0; e < F::V; ++e) {
         x[e] = cscale(cmulc(u[e], pw[e]), c);                // conj(c_it s~^(-1/2-it)) * u
         pw[e] = cmul(pw[e], inv[e]);
       }
-      F::run(x, wl, twl, lane);
-      float2* W = a.W + (size_t)(it - 1) * a.wstride;
+      F::template run<false>(x, line, twl, w.l);
+      const RowBuf<N, T> W(a.W + (size_t)(it - 1) * a.wstride, w, a.quad != 0);
 #pragma unroll
-      for (int e = 0; e < C::V; ++e) {
-        int b, i;
-        edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-        const int lr = rb + b;
-        if (lr < nrows) W[widx(a, lr, i, N)] = to_f2(cscale(x[e], a.scale));
-      }
+      for (int e = 0; e < F::V; ++e) W.store(to_f2(cscale(x[e], (S)a.scale)), F::last_c(e));
     }
   }
 }
@@ -422,69 +309,58 @@ __global__ __launch_bounds__(kThreads) void k_rows_scatter_adj(KArgs a) {
 //             reference's ic_adj uses float atomicAdd, imaging_condition.cu:103-104).
 // IC = false: out = (add ? out : 0) + x  (standalone Scatter adjoint).
 template <int N, bool IC, bool MAP, class T = float2>
-__global__ __launch_bounds__(kThreads) void k_rows_adj_out(KArgs a) {
-  using C = BRowCfg<N>;
+__global__ __launch_bounds__(kRowThreads) void k_rows_adj_out(KArgs a) {
+  using F = LaneFft<N, T>;
   using S = real_of<T>;
-  using Fi = WaveFft<N, C::NB, false, true, PadLds<N>, T>;
-  __shared__ T lds[kWaves * C::LDSW];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nrows = a.np * a.NY;
-  const int rb = (blockIdx.x * kWaves + wave) * C::NB;
-  // twiddles in LDS: a global twiddle load would wait (one counter for all
-  // vector memory operations) for every load still in flight
-  __shared__ T twl[N];
-  const T* twg = twx_of(a, (T*)nullptr);
-  for (int i = threadIdx.x; i < N; i += kThreads) twl[i] = twg[i];
+  __shared__ T lds[kRowWaves * F::NB * F::STRIDE];
+  __shared__ T twl[F::TW];
+  const RowLane<N, T> w(a);
+  T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
+  // the imaging condition writes the model region only: rows of the
+  // padding (y >= ny) have nothing to produce, not even their transform
+  const bool any = IC ? wave_in_model<N>(a, w) : !w.empty();
+  T x[F::V];
+#pragma unroll
+  for (int e = 0; e < F::V; ++e) x[e] = cz<T>();
+  if (any && a.nterm > 1) {
+    const RowBuf<N, T> K(a.K, w, a.quad != 0);
+#pragma unroll
+    for (int e = 0; e < F::V; ++e) x[e] = from_f2<T>(K.load(F::last_c(e)));
+  }
+  row_twiddles<N>(twl, twx_of(a, (T*)nullptr));
   __syncthreads();
-  if (rb >= nrows) return;
+  if (!any) return;
+  if (a.nterm > 1) F::template run<true>(x, line, twl, w.l);
+  const S h = (S)(0.5f * a.w[w.iw] * a.dz);
+  const float2* slow = slow_row(a, model_iw<MAP>(a, w.iw), w.iy);
+  const RowBuf<N, T> in(a.in, w, false);
+  const int nin = IC ? (w.live && w.iy < a.ny ? a.nx : 0) : N;  // columns that are used
+  auto value = [&](int e) {
+    T rsq, inv;
+    scatter_factors(a, slow_at(a, slow, w.l + F::first_c(e)), rsq, inv);
+    const T d = from_f2<T>(in.load_if(w.l + F::first_c(e) < nin, F::first_c(e)));
+    const T u = CX<T>::mk(-h * d.y, h * d.x);
+    return cadd(cscale(x[e], (S)a.scale), cmulc(u, rsq));
+  };
   if constexpr (IC) {
-    // the imaging condition writes the model region only: rows of the
-    // padding (y >= ny) have nothing to produce, not even their transform
-    bool any = false;
-    for (int b = 0; b < C::NB; ++b) {
-      const int lr = rb + b;
-      if (lr < nrows && lr % a.NY < a.ny) any = true;
-    }
-    if (!any) return;
-  }
-  T x[C::V];
-  if (a.nterm > 1) {
+    const RowBuf<N, T> bg(a.bg, w, false);
+    float2* aux = a.aux + (size_t)(w.iw * a.ny + (w.iy < a.ny ? w.iy : 0)) * a.nx;
+    const int nx = nin;
+    in_groups<F>(x, a.nx, [&](int e) {
+      const int i = w.l + F::first_c(e);
+      const float2 old = a.add ? aux[i < nx ? i : 0] : czero();
+      const T g = cmulc(value(e), from_f2<T>(bg.load_if(i < nx, F::first_c(e))));
+      return a.add ? cadd(from_f2<T>(old), g) : g;
+    });
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, Fi::P::first(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      x[e] = lr < nrows ? from_f2<T>(a.K[widx(a, lr, i, N)]) : cz<T>();
-    }
-    Fi::run(x, lds + wave * C::LDSW, twl, lane);
+    for (int e = 0; e < F::V; ++e)
+      if (w.l + F::first_c(e) < nx) aux[w.l + F::first_c(e)] = to_f2(x[e]);
   } else {
+    const RowBuf<N, T> out(a.out, w, false);
 #pragma unroll
-    for (int e = 0; e < C::V; ++e) x[e] = cz<T>();
-  }
-#pragma unroll
-  for (int e = 0; e < C::V; ++e) {
-    int b, i;
-    edge_pos<N, C::NB, Fi::P::last(), false>(lane, e, b, i);
-    const int lr = rb + b;
-    if (lr < nrows) {
-      const int p = lr / a.NY, iy = lr - p * a.NY;
-      const int iw = plane_iw(a, p);
-      const unsigned idx = lr * N + i;
-      T rsq, inv;
-      scatter_factors(a, model_iw<MAP>(a, iw), iy, i, rsq, inv);
-      const S h = (S)(0.5f * a.w[iw] * a.dz);
-      const T d = from_f2<T>(a.in[idx]);
-      const T u = CX<T>::mk(-h * d.y, h * d.x);
-      const T y = cadd(cscale(x[e], a.scale), cmulc(u, rsq));
-      if constexpr (IC) {
-        if (iy < a.ny && i < a.nx) {
-          const unsigned m = (iw * a.ny + iy) * a.nx + i;
-          const T g = cmulc(y, from_f2<T>(a.bg[idx]));
-          a.aux[m] = to_f2(a.add ? cadd(from_f2<T>(a.aux[m]), g) : g);
-        }
-      } else {
-        a.out[idx] = to_f2(a.add ? cadd(from_f2<T>(a.out[idx]), y) : y);
-      }
+    for (int e = 0; e < F::V; ++e) {
+      const T y = value(e);
+      out.store(to_f2(a.add ? cadd(from_f2<T>(out.load(F::first_c(e))), y) : y), F::first_c(e));
     }
   }
 }
@@ -707,21 +583,6 @@ __global__ __launch_bounds__(kThreads) void k_plane_sum(const float2* __restrict
 }
 
 // ------------------------------------------------------------------ launchers
-template <class Fn>
-static hipError_t bdispatch(int n, Fn&& fn) {
-  switch (n) {
-#define CASE(S) case S: return fn(std::integral_constant<int, S>{});
-    CASE(8) CASE(12) CASE(16) CASE(24) CASE(32) CASE(48) CASE(64) CASE(96) CASE(128) CASE(192)
-    CASE(256) CASE(384) CASE(512) CASE(768) CASE(1024)
-#undef CASE
-    default: return hipErrorInvalidValue;
-  }
-}
-static dim3 brow_grid(int N, int nrows) {
-  const int nb = row_nb(N);
-  const int waves = (nrows + nb - 1) / nb;
-  return dim3((waves + kWaves - 1) / kWaves);
-}
 static inline dim3 bflat(long long n) {
   long long g = (n + kThreads - 1) / kThreads;
   if (g > (1ll << 30)) g = 1ll << 30;
@@ -735,19 +596,20 @@ static inline dim3 bflat(long long n) {
 // the fused Born forms only).
 template <template <int, bool, bool, class> class K, bool FLAG, bool F64 = false>
 static hipError_t launch_mapped(const KArgs& a, hipStream_t st) {
-  return bdispatch(a.NX, [&](auto nc) -> hipError_t {
+  return dispatch_n(a.NX, [&](auto nc) -> hipError_t {
     constexpr int N = decltype(nc)::value;
-    const dim3 g = brow_grid(N, a.np * a.NY);
+    const dim3 g = row_grid<N, float2>(a.np * a.NY);
     if constexpr (F64) {
       if (a.f64) {
-        if (a.mplane) hipLaunchKernelGGL((K<N, FLAG, true, double2>::fn), g, dim3(kThreads), 0, st, a);
-        else hipLaunchKernelGGL((K<N, FLAG, false, double2>::fn), g, dim3(kThreads), 0, st, a);
+        const dim3 g64 = row_grid<N, double2>(a.np * a.NY);
+        if (a.mplane) hipLaunchKernelGGL((K<N, FLAG, true, double2>::fn), g64, dim3(kRowThreads), 0, st, a);
+        else hipLaunchKernelGGL((K<N, FLAG, false, double2>::fn), g64, dim3(kRowThreads), 0, st, a);
         return hipGetLastError();
       }
     }
     if (a.f64) return hipErrorInvalidValue;
-    if (a.mplane) hipLaunchKernelGGL((K<N, FLAG, true, float2>::fn), g, dim3(kThreads), 0, st, a);
-    else hipLaunchKernelGGL((K<N, FLAG, false, float2>::fn), g, dim3(kThreads), 0, st, a);
+    if (a.mplane) hipLaunchKernelGGL((K<N, FLAG, true, float2>::fn), g, dim3(kRowThreads), 0, st, a);
+    else hipLaunchKernelGGL((K<N, FLAG, false, float2>::fn), g, dim3(kRowThreads), 0, st, a);
     return hipGetLastError();
   });
 }

@@ -124,11 +124,20 @@ static std::vector<double2> twiddle_table64(int n) {  // exp(-2 pi i k / n) in d
   }
   return t;
 }
-static std::vector<float2> twiddle_table(int n) {  // the float64 table rounded once
-  std::vector<float2> t(n);
-  const auto t64 = twiddle_table64(n);
-  for (int k = 0; k < n; ++k) t[k] = make_float2((float)t64[k].x, (float)t64[k].y);
+// the row transforms' stage twiddles (twiddle_exp) of the float32 or float64 plan, in double
+static std::vector<double2> stage_twiddles(int n, bool f64) {
+  const auto t = twiddle_table64(n);
+  std::vector<double2> o(n);
+  for (int i = 0; i < n; ++i) o[i] = t[twiddle_exp(n, f64, i)];
+  return o;
+}
+static std::vector<float2> rounded(const std::vector<double2>& t64) {
+  std::vector<float2> t(t64.size());
+  for (size_t k = 0; k < t.size(); ++k) t[k] = make_float2((float)t64[k].x, (float)t64[k].y);
   return t;
+}
+static std::vector<float2> twiddle_table(int n) {  // the float64 table rounded once
+  return rounded(twiddle_table64(n));
 }
 
 void validate_dims(const fwix_dims* d, bool need_fft) {
@@ -172,10 +181,10 @@ void Tables::init(const fwix_dims& d, int tx, int ty) {
   upload_bytes(b_tapx, tx_.data(), tx_.size() * 4);
   upload_bytes(b_tapy, ty_.data(), ty_.size() * 4);
   if (fft_size_supported(d.NX) && fft_size_supported(d.NY)) {
-    auto twx = twiddle_table(d.NX), twy = twiddle_table(d.NY);
+    auto twx = rounded(stage_twiddles(d.NX, false)), twy = twiddle_table(d.NY);
     upload_bytes(b_twx, twx.data(), twx.size() * 8);
     upload_bytes(b_twy, twy.data(), twy.size() * 8);
-    auto twx64 = twiddle_table64(d.NX), twy64 = twiddle_table64(d.NY);
+    auto twx64 = stage_twiddles(d.NX, true), twy64 = twiddle_table64(d.NY);
     upload_bytes(b_twx64, twx64.data(), twx64.size() * 16);
     upload_bytes(b_twy64, twy64.data(), twy64.size() * 16);
   }

@@ -167,6 +167,69 @@ template <bool INV> struct Dft<8, INV> {
   }
 };
 
+// 16 = 4 x 4; the twiddles between the two layers are multiples of pi/8
+template <bool INV> struct Dft<16, INV> {
+  template <class T>
+  __device__ __forceinline__ static void run(T* x) {
+    using S = real_of<T>;
+    const S r = (S)0.70710678118654752440, c = (S)0.92387953251128675613, s = (S)0.38268343236508977173;
+    T y[4][4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+#pragma unroll
+      for (int a = 0; a < 4; ++a) y[b][a] = x[4 * a + b];
+      Dft<4, INV>::run(y[b]);
+    }
+    auto rot = [&](T v, S cr, S si) {  // v * (cr + sgn i si), sgn = -1 forward
+      return INV ? cmul(v, CX<T>::mk(cr, si)) : cmulc(v, CX<T>::mk(cr, si));
+    };
+    auto w2 = [&](T v) { return cscale(cadd(v, mul_si<INV>(v)), r); };       // pi/4
+    auto w6 = [&](T v) { return cscale(csub(mul_si<INV>(v), v), r); };       // 3 pi/4
+    y[1][1] = rot(y[1][1], c, s);   y[1][2] = w2(y[1][2]);           y[1][3] = rot(y[1][3], s, c);
+    y[2][1] = w2(y[2][1]);          y[2][2] = mul_si<INV>(y[2][2]);  y[2][3] = w6(y[2][3]);
+    y[3][1] = rot(y[3][1], s, c);   y[3][2] = w6(y[3][2]);           y[3][3] = rot(y[3][3], -c, -s);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      T z[4] = {y[0][k], y[1][k], y[2][k], y[3][k]};
+      Dft<4, INV>::run(z);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) x[k + 4 * d] = z[d];
+    }
+  }
+};
+
+// R = A * B with coprime A, B by the prime-factor map, free of twiddles:
+// input n = (B n1 + A n2) mod R, output k with k mod A = k1, k mod B = k2
+template <int A, int B, bool INV> struct DftPfa {
+  static constexpr int R = A * B;
+  static constexpr int crt(int k1, int k2) {
+    for (int k = 0; k < R; ++k)
+      if (k % A == k1 && k % B == k2) return k;
+    return 0;
+  }
+  template <class T>
+  __device__ __forceinline__ static void run(T* x) {
+    T y[A][B];  // [n1][k2]
+#pragma unroll
+    for (int n1 = 0; n1 < A; ++n1) {
+#pragma unroll
+      for (int n2 = 0; n2 < B; ++n2) y[n1][n2] = x[(B * n1 + A * n2) % R];
+      Dft<B, INV>::run(y[n1]);
+    }
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) {
+      T z[A];
+#pragma unroll
+      for (int n1 = 0; n1 < A; ++n1) z[n1] = y[n1][k2];
+      Dft<A, INV>::run(z);
+#pragma unroll
+      for (int k1 = 0; k1 < A; ++k1) x[crt(k1, k2)] = z[k1];
+    }
+  }
+};
+template <bool INV> struct Dft<6, INV> : DftPfa<3, 2, INV> {};
+template <bool INV> struct Dft<12, INV> : DftPfa<3, 4, INV> {};
+
 // ----------------------------------------------------------------- wave ordering
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -276,6 +339,265 @@ struct WaveFft {
     asm volatile("" ::: "memory");
     asm volatile("" : "+v"(lane));
     stages<0>(v, lds, tw, lane);
+  }
+};
+
+// ================================================================= lane transform
+// The transforms of the row passes.  L = N / V lanes hold one line of N
+// points, V values each, and a wave holds 64 / L lines; lane l of a line owns
+// the butterflies j = l + L q of every stage.  The plans below take few,
+// wide stages (their count is what sets the LDS exchanges), with V a multiple
+// of every radix and L a divisor (or a multiple) of every sub-transform
+// length, so that every position, LDS address and twiddle index of a value is
+// a per-lane base plus a compile-time constant: the loops carry no index
+// arithmetic (the transforms it replaced spent half of their VALU
+// instructions on it).
+//
+//   forward stage s (radix R, sub-transform length Ns): butterfly j reads
+//     positions j + r N/R, multiplies by W_{Ns R}^(r (j mod Ns)), and leaves
+//     output r at position (j / Ns) Ns R + j mod Ns + r Ns
+//   inverse: the forward stages undone in reverse order (butterfly, then the
+//     conjugate twiddles, exchanges written where the forward reads and read
+//     where it writes), so it starts at the positions the forward ends at and
+//     ends where the forward starts.
+struct PlanDef {
+  int V, S, R[4];
+};
+// Short lines take narrow plans (V <= 12): their launches are small and more
+// waves in flight are worth more than a stage less (256 points: Born adjoint
+// rows 21.3 us at V = 16, two stages, 17.5 us at V = 8, three).  The long
+// lines with a factor 3 take V = 24 (768 points: 4 stages of V = 12 against 3);
+// float64 lines hold at most 16 values per lane (twice the registers each).
+__host__ __device__ constexpr PlanDef plan_def(int N, bool f64) {
+  switch (N) {
+    case 8: return {4, 2, {4, 2}};
+    case 12: return {12, 1, {12}};
+    case 16: return {4, 2, {4, 4}};
+    case 24: return {12, 2, {4, 6}};
+    case 32: return {8, 2, {8, 4}};
+    case 48: return {12, 2, {4, 12}};
+    case 64: return {8, 2, {8, 8}};
+    case 96: return {12, 3, {4, 2, 12}};
+    case 128: return {8, 3, {8, 4, 4}};
+    case 192: return {12, 3, {4, 4, 12}};
+    case 256: return {8, 3, {8, 8, 4}};
+    case 384: return f64 ? PlanDef{12, 4, {4, 4, 4, 6}} : PlanDef{24, 3, {8, 8, 6}};
+    case 512: return {8, 3, {8, 8, 8}};
+    case 768: return f64 ? PlanDef{12, 4, {4, 4, 4, 12}} : PlanDef{24, 3, {8, 8, 12}};
+    case 1024: return {16, 3, {16, 8, 8}};
+    default: return {0, 0, {}};
+  }
+}
+__host__ __device__ constexpr int plan_ns(const PlanDef& d, int s) {
+  int p = 1;
+  for (int k = 0; k < s; ++k) p *= d.R[k];
+  return p;
+}
+// Entry i of a length's twiddle table: the exponent e of exp(-2 pi i e / N).
+// Stage s holds its R - 1 rows of Ns factors one after another ([r][k], k
+// fastest), so a lane reads W^(rk) at a base of its own plus r Ns, neighbouring
+// lanes on neighbouring entries.  Entries past the last stage's are zero.
+__host__ __device__ constexpr int twiddle_exp(int N, bool f64, int i) {
+  const PlanDef d = plan_def(N, f64);
+  int o = 0;
+  for (int s = 1; s < d.S; ++s) {
+    const int Ns = plan_ns(d, s), n = (d.R[s] - 1) * Ns;
+    if (i < o + n) {
+      const int r = (i - o) / Ns + 1, k = (i - o) % Ns;
+      return r * k * (N / (Ns * d.R[s]));
+    }
+    o += n;
+  }
+  return 0;
+}
+
+template <int N, class T = float2>
+struct LaneFft {
+  // (a constexpr array member would be a device constant, loaded at run time:
+  // the plan is only ever read through these functions)
+  static constexpr bool F64 = sizeof(T) == 16;
+  static constexpr int V = plan_def(N, F64).V, S = plan_def(N, F64).S, L = N / V, NB = 64 / L;
+  static_assert(V > 0 && L * V == N && NB * L == 64, "lanes must divide the line and the wave");
+  static constexpr int R(int s) { return plan_def(N, F64).R[s]; }
+  static constexpr int Ns(int s) { return plan_ns(plan_def(N, F64), s); }
+  static constexpr int tw_off(int s) {
+    int o = 0;
+    for (int k = 1; k < s; ++k) o += (R(k) - 1) * Ns(k);
+    return o;
+  }
+  static constexpr int TW = tw_off(S) > 0 ? tw_off(S) : 1;  // table entries (N - R(0))
+
+  // Padding of the exchange between stages s and s + 1, in positions: Ns more
+  // after each block of G, but none where the sum reaches a row of banks (32).
+  // 32 lanes then write runs of Ns positions NsR apart to distinct banks,
+  // and still read 32 consecutive positions without a gap.
+  static constexpr int G(int s) {
+    int g = R(s) * Ns(s);
+    while (g < 32) g *= 2;
+    return g;
+  }
+  static constexpr int WR(int s) { return Ns(s) >= 32 ? 1 : 32 / Ns(s); }
+  __host__ __device__ static constexpr int pad(int s, int blk) {
+    const unsigned b = (unsigned)blk, w = (unsigned)WR(s);
+    return (int)(b % w + b / w * (w - 1)) * Ns(s);
+  }
+  static constexpr int stride_min() {
+    int m = N;
+    for (int s = 0; s + 1 < S; ++s) {
+      const int p = pad(s, (N - 1) / G(s));
+      if (N + p > m) m = N + p;
+    }
+    return m;
+  }
+  // lines of a wave: short lines side by side in the banks (stride = L mod
+  // 32); the others 8 past a multiple of 32, so that four rows staged as
+  // quads fall into distinct banks
+  static constexpr int STRIDE = stride_min() + ((L < 32 ? L : 8) + 32 * 64 - stride_min() % 32) % 32;
+
+  // position of value v of lane l before the first forward stage (= after the
+  // inverse) and after the last (= before the inverse): lane base + constant
+  static constexpr int in_c(int s, int v) { return L * (v / R(s)) + (v % R(s)) * (N / R(s)); }
+  static constexpr int first_c(int v) { return in_c(0, v); }
+  static constexpr int last_c(int v) { return in_c(S - 1, v); }
+
+  // exchange after stage s: LDS offset of value v where stage s + 1 reads
+  // (IN) and where stage s wrote (OUT), as a lane base and a constant
+  template <int s>
+  __device__ __forceinline__ static int in_base(int l) {
+    return l + pad(s, (int)((unsigned)l / (unsigned)G(s)));
+  }
+  template <int s>
+  static constexpr int in_const(int v) {
+    const int C = in_c(s + 1, v);
+    return C + pad(s, C / G(s));
+  }
+  template <int s>
+  static constexpr bool in_ok() {
+    for (int v = 0; v < V; ++v) {
+      const int C = in_c(s + 1, v);
+      // the lane part stays in its block, or the constant is whole blocks
+      // and the sum of the block numbers adds no bank row of its own
+      const int blk = C / G(s), span = (L - 1) / G(s);
+      if (!(C % G(s) + L <= G(s) || (C % G(s) == 0 && (blk % WR(s) == 0 || blk % WR(s) + span < WR(s)))))
+        return false;
+    }
+    return true;
+  }
+  template <int s>
+  __device__ __forceinline__ static int out_base(int l) {
+    constexpr int n = Ns(s), g = G(s) / (n * R(s));
+    const unsigned a = (unsigned)l / (unsigned)n;
+    return (int)(a * n * R(s) + (unsigned)l % (unsigned)n) + pad(s, (int)(a / g));
+  }
+  template <int s>
+  static constexpr int out_const(int v) {
+    constexpr int n = Ns(s), g = G(s) / (n * R(s));
+    const int q = v / R(s), r = v % R(s);
+    return q * L * R(s) + r * n + pad(s, q * (L / n) / g);
+  }
+  template <int s>
+  static constexpr bool out_ok() {
+    constexpr int n = Ns(s), g = G(s) / (n * R(s));
+    if (L % n) return false;
+    for (int q = 0; q < V / R(s); ++q) {
+      const int a = q * (L / n), span = (L / n - 1) / g;  // blocks the lane part reaches past the constant's
+      const bool whole = a % g == 0 || a % g + L / n <= g;
+      if (!whole) return false;
+      if ((a / g) % WR(s) != 0 && (a / g) % WR(s) + span >= WR(s)) return false;
+    }
+    return true;
+  }
+
+  template <int s, bool INV>
+  __device__ __forceinline__ static void twiddle(T* v, const T* __restrict__ tw, int l) {
+    if constexpr (s > 0) {
+      constexpr int n = Ns(s);
+      static_assert(L % n == 0 || n % L == 0, "a lane's twiddles must sit at constant offsets");
+      const T* t = tw + tw_off(s) + (L % n == 0 ? (int)((unsigned)l % (unsigned)n) : l);
+#pragma unroll
+      for (int q = 0; q < V / R(s); ++q) {
+        const int kc = L % n == 0 ? 0 : (L * q) % n;
+#pragma unroll
+        for (int r = 1; r < R(s); ++r) {
+          const T w = t[(r - 1) * n + kc];
+          T& x = v[q * R(s) + r];
+          x = INV ? cmulc(x, w) : cmul(x, w);
+        }
+      }
+    }
+  }
+  template <int s, bool INV>
+  __device__ __forceinline__ static void butterflies(T* v) {
+#pragma unroll
+    for (int q = 0; q < V / R(s); ++q) Dft<R(s), INV>::run(v + q * R(s));
+  }
+  template <int s>
+  __device__ __forceinline__ static void put_out(const T* v, T* line, int l) {
+    static_assert(out_ok<s>(), "exchange positions must split into lane base and constant");
+    T* p = line + out_base<s>(l);
+#pragma unroll
+    for (int e = 0; e < V; ++e) p[out_const<s>(e)] = v[e];
+  }
+  template <int s>
+  __device__ __forceinline__ static void get_out(T* v, const T* line, int l) {
+    const T* p = line + out_base<s>(l);
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[e] = p[out_const<s>(e)];
+  }
+  template <int s>
+  __device__ __forceinline__ static void put_in(const T* v, T* line, int l) {
+    static_assert(in_ok<s>(), "exchange positions must split into lane base and constant");
+    T* p = line + in_base<s>(l);
+#pragma unroll
+    for (int e = 0; e < V; ++e) p[in_const<s>(e)] = v[e];
+  }
+  template <int s>
+  __device__ __forceinline__ static void get_in(T* v, const T* line, int l) {
+    const T* p = line + in_base<s>(l);
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[e] = p[in_const<s>(e)];
+  }
+
+  // stages FROM .. TO - 1 of the forward transform, with the exchanges between
+  // them (through this line's own LDS: wave ordering is enough)
+  template <int FROM, int TO>
+  __device__ __forceinline__ static void forward(T* v, T* line, const T* __restrict__ tw, int l) {
+    if constexpr (FROM < TO) {
+      twiddle<FROM, false>(v, tw, l);
+      butterflies<FROM, false>(v);
+      if constexpr (FROM + 1 < TO) {
+        put_out<FROM>(v, line, l);
+        wave_sync();
+        get_in<FROM>(v, line, l);
+        wave_sync();
+        forward<FROM + 1, TO>(v, line, tw, l);
+      }
+    }
+  }
+  // stages FROM - 1 .. TO of the inverse
+  template <int FROM, int TO>
+  __device__ __forceinline__ static void inverse(T* v, T* line, const T* __restrict__ tw, int l) {
+    if constexpr (FROM > TO) {
+      butterflies<FROM - 1, true>(v);
+      twiddle<FROM - 1, true>(v, tw, l);
+      if constexpr (FROM - 1 > TO) {
+        put_in<FROM - 2>(v, line, l);
+        wave_sync();
+        get_out<FROM - 2>(v, line, l);
+        wave_sync();
+        inverse<FROM - 1, TO>(v, line, tw, l);
+      }
+    }
+  }
+  // Whole transforms of a line held by one wave, unnormalized: v at
+  // first_c / last_c positions in, at last_c / first_c out.  The memory
+  // clobber keeps the twiddle loads next to their use (hoisted out of a
+  // per-reference loop they would cost two registers each).
+  template <bool INV>
+  __device__ __forceinline__ static void run(T* v, T* line, const T* __restrict__ tw, int l) {
+    asm volatile("" ::: "memory");
+    if constexpr (INV) inverse<S, 0>(v, line, tw, l);
+    else forward<0, S>(v, line, tw, l);
   }
 };
 

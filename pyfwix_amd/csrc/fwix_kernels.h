@@ -8,11 +8,12 @@ namespace fwix {
 // Supported lateral FFT sizes: 2^a and 3*2^a between 8 and 1024.
 constexpr bool size_has3(int N) { return N % 3 == 0; }
 
-// Rows per wavefront in the row passes (V = NB*N/64 values per lane).
-constexpr int row_nb(int N) {
-  const int base = size_has3(N) ? 768 : 512;
-  return N >= base ? 1 : base / N;
-}
+// Row passes: workgroups of 4 waves, each with LaneFft::NB rows (64 / NB lanes a
+// row).  (8 waves to share one twiddle table at 1024 points, 16 waves per CU
+// instead of 12, cap the registers at 128: the chained select pass spills and
+// takes 1298 instead of 824 us per 128-plane launch.)
+constexpr int kRowWaves = 4;
+constexpr int kRowThreads = 64 * kRowWaves;
 // Column passes: 512-thread workgroups, 8 waves x CW/8 columns, with each
 // lane holding V = CW*N/512 values: 8 (2^a, N <= 512), 16 (1024) or 12 (3*2^a).
 // Two workgroups fit a CU, so one tile's loads overlap another's transforms.
@@ -38,7 +39,6 @@ constexpr int col_cw(int N) {
 }
 constexpr int kColThreads = 512;
 constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
 
 // LDS layouts -------------------------------------------------------------
 // Stockham exchanges write with stride R inside a batch; one pad slot every
@@ -66,10 +66,10 @@ struct KArgs {
   const float* w;          // (NW) 2 pi f
   const float* tapx;       // (NX) taper weights
   const float* tapy;       // (NY)
-  const float2* twx;       // (NX) twiddles exp(-2 pi i k/NX)
-  const float2* twy;       // (NY)
-  const double2* twx64;    // (NX), (NY) twiddles and taper weights in float64, for
-  const double2* twy64;    //   the passes that run in float64 arithmetic (f64)
+  const float2* twx;       // (NX) stage twiddles of the row transforms (twiddle_exp)
+  const float2* twy;       // (NY) twiddles exp(-2 pi i k/NY)
+  const double2* twx64;    // the same tables and taper weights in float64, for the
+  const double2* twy64;    //   passes that run in float64 arithmetic (f64)
   const double* tapx64;
   const double* tapy64;
   const float2* slow;      // (NW, ny, nx) unpadded slowness slice (Born scatter)
@@ -134,6 +134,130 @@ __device__ __forceinline__ int model_iw(const KArgs& a, int iw) {
 }
 // once-per-workgroup form (column kernels)
 __device__ __forceinline__ int model_iw_any(const KArgs& a, int iw) { return a.mplane ? a.mplane[iw] : iw; }
+
+// The rows of one wave of a row pass, as one lane sees them: row rb + b of the
+// chunk, at lane l of its LaneFft::L lanes.  Rows at or beyond nrows (the last
+// wave's) are computed on zeros and never stored.
+template <int N, class T>
+struct RowLane {
+  using F = LaneFft<N, T>;
+  int l, b, rb, nrows;
+  bool live;
+  int iw, iy;  // frequency plane and row of the plane (of the last row for dead lanes)
+  __device__ __forceinline__ explicit RowLane(const KArgs& a) {
+    const int lane = (int)threadIdx.x & 63;
+    l = (int)((unsigned)lane % F::L);
+    b = (int)((unsigned)lane / F::L);
+    nrows = a.np * a.NY;
+    rb = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * kRowWaves + (threadIdx.x >> 6)) * F::NB));
+    const int lr = rb + b;
+    live = lr < nrows;
+    const int row = live ? lr : nrows - 1;
+    const int p = row / a.NY;
+    iy = row - p * a.NY;
+    iw = plane_iw(a, p);
+  }
+  __device__ __forceinline__ bool empty() const { return rb >= nrows; }  // wave-uniform
+};
+// The wave's rows of a wavefield (row-major) or of the K / W scratch (in the
+// launch's layout) as a buffer resource: a lane's elements sit at one 32-bit
+// lane offset plus a uniform offset per element, so they cost no address
+// arithmetic, and the hardware range check reads zero / drops stores of
+// rows beyond the last.
+template <int N, class T>
+struct RowBuf {
+  using F = LaneFft<N, T>;
+  __amdgpu_buffer_rsrc_t r;
+  unsigned v, row;
+  int cs, l;
+  __device__ __forceinline__ RowBuf(const float2* base, const RowLane<N, T>& w, bool quad) : l(w.l) {
+    const int r0 = quad ? w.rb & ~3 : w.rb;
+    const int left = w.nrows - r0, most = F::NB + 4;
+    const int rows = left < 0 ? 0 : left < most ? left : most;
+    r = __builtin_amdgcn_make_buffer_rsrc((void*)(base + (size_t)r0 * N), (short)0,
+                                          __builtin_amdgcn_readfirstlane(rows * N * 8), 0x00020000);
+    const unsigned y = (unsigned)(w.rb - r0 + w.b);
+    row = quad ? ((y >> 2) * N + (y & 3)) * 32u : y * N * 8u;
+    v = row + (quad ? (((unsigned)l >> 2) << 4) + ((unsigned)l & 3u) : (unsigned)l) * 8u;
+    cs = quad ? 32 : 8;
+  }
+  // column l + C (C a compile-time constant after unrolling)
+  __device__ __forceinline__ unsigned voff(int C) const {
+    if constexpr (F::L % 4 == 0) return v;
+    const unsigned x = (unsigned)(l + C);
+    return cs == 32 ? row + (((x >> 2) << 4) + (x & 3u)) * 8u : row + x * 8u;
+  }
+  __device__ __forceinline__ int soff(int C) const { return F::L % 4 == 0 ? C * cs : 0; }
+  __device__ __forceinline__ float2 load(int C) const {
+    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff(C), soff(C), 0));
+  }
+  // where the lane's condition holds, else zero without touching memory: every
+  // element's load is in flight at once, which a branch around each would forbid
+  __device__ __forceinline__ float2 load_if(bool on, int C) const {
+    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, on ? (int)voff(C) : (int)0x80000000u, soff(C), 0));
+  }
+  __device__ __forceinline__ void store(float2 x, int C) const {
+    using U2 = __attribute__((ext_vector_type(2))) unsigned;
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, x), r, (int)voff(C), soff(C), 0);
+  }
+};
+// x[e] = f(e) for the elements of a lane, in groups: a group's loads are in
+// flight together, and its results are formed before the next group's loads
+// are issued, which bounds the registers that loads of several arrays take at
+// once (left alone the compiler issues every element's loads first).
+// A group holds the elements at positions from r0 N / R(0) on (first_c order),
+// and groups that start at or beyond column `cols` are skipped: nothing of
+// theirs is needed (the padding of an imaging or scattering source).
+__device__ __forceinline__ void pin(float2& x) { asm volatile("" : "+v"(x.x), "+v"(x.y) : : "memory"); }
+__device__ __forceinline__ void pin(double2& x) { asm volatile("" : "+v"(x.x), "+v"(x.y) : : "memory"); }
+template <class F, class T, class Fn>
+__device__ __forceinline__ void in_groups(T* x, int cols, Fn&& f) {
+  constexpr int R = F::R(0), Q = F::V / R, most = sizeof(T) == 16 || F::V == 16 ? 4 : 8;
+  constexpr int G = Q >= most ? 1 : most / Q < R ? most / Q : R;  // butterfly inputs per group
+#pragma unroll
+  for (int r0 = 0; r0 < R; r0 += G) {
+    if (r0 * (F::L * Q) < cols) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int r = r0; r < (r0 + G < R ? r0 + G : R); ++r) x[q * R + r] = f(q * R + r);
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int r = r0; r < (r0 + G < R ? r0 + G : R); ++r) pin(x[q * R + r]);
+  }
+}
+// labels of a lane's elements, four to a register
+template <int V>
+struct Labels {
+  uint32_t w[(V + 3) / 4];
+  template <class Pos>
+  __device__ __forceinline__ void load(const uint8_t* __restrict__ p, Pos&& pos) {
+#pragma unroll
+    for (int k = 0; k < (V + 3) / 4; ++k) w[k] = 0;
+#pragma unroll
+    for (int e = 0; e < V; ++e) w[e / 4] |= (uint32_t)p[pos(e)] << (8 * (e % 4));
+  }
+  __device__ __forceinline__ int at(int e) const { return (int)((w[e / 4] >> (8 * (e % 4))) & 255u); }
+};
+// this workgroup's copy of the row transforms' twiddle table; the caller
+// synchronises.  In LDS because a global load inside the term loops would
+// wait (one counter for all vector memory operations) for the term's
+// stores or the next term's loads still in flight.
+template <int N, class T>
+__device__ __forceinline__ void row_twiddles(T* twl, const T* __restrict__ tw) {
+  for (int i = threadIdx.x; i < LaneFft<N, T>::TW; i += kRowThreads) twl[i] = tw[i];
+}
+// references present in any row of this wave (all bits when there are no masks)
+template <int N, class T, bool MAP>
+__device__ __forceinline__ uint32_t wave_row_mask(const KArgs& a, const RowLane<N, T>& w) {
+  if (!a.rowmask) return 0xffffffffu;
+  uint32_t m = a.rowmask[model_iw<MAP>(a, w.iw) * a.NY + w.iy];
+#pragma unroll
+  for (int o = LaneFft<N, T>::L; o < 64; o <<= 1) m |= (uint32_t)__shfl_xor((int)m, o);
+  return __builtin_amdgcn_readfirstlane(m);
+}
 
 // lowest set bit of m above position r (32 when none); r = -1 gives the lowest
 __device__ __forceinline__ int next_bit(uint32_t m, int r) {

@@ -4,8 +4,27 @@
 #include <stdint.h>
 #include "fwix_kernels.h"
 
+#include <type_traits>
+
 namespace fwix {
 
+#define FWIX_SIZES(X) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(1024)
+
+template <class Fn>
+hipError_t dispatch_n(int n, Fn&& fn) {
+  switch (n) {
+#define CASE(S) case S: return fn(std::integral_constant<int, S>{});
+    FWIX_SIZES(CASE)
+#undef CASE
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int N, class T>
+inline dim3 row_grid(int nrows) {
+  constexpr int per = kRowWaves * LaneFft<N, T>::NB;
+  return dim3((nrows + per - 1) / per);
+}
 // Argument block of the point-wise operator kernels.
 struct PwArgs {
   int NX, NY, NW, NS;

@@ -9,9 +9,7 @@
 //   NSPS adjoint   (corrected; NSPS.cpp:6-25 passes swapped arguments)
 //     rows_fwd             ->  cols_fanout(Phi_r^adj) -> rows_select
 //
-// Rows are transformed one wavefront per row (or per few short rows), loaded
-// and stored straight from/to HBM in the positions the first/last Stockham
-// stage needs.  Columns are staged through a [NY][CW+1] LDS tile so global
+// Row passes: row_kernels.hip.  Columns are staged through a [NY][CW+1] LDS tile so global
 // accesses stay 128-byte coalesced.  The per-reference fan-out keeps the
 // spectrum of a column tile in registers and runs all nref inverse
 // transforms from it; the fan-in accumulates all nref spectra in registers
@@ -23,12 +21,6 @@
 
 namespace fwix {
 
-template <int N>
-struct RowCfg {
-  static constexpr int NB = row_nb(N);
-  static constexpr int V = NB * N / 64;
-  static constexpr int LDSW = NB * padded(N);
-};
 // Column passes: 16 waves x NB columns.  The [N][CW+1] tile that stages the
 // coalesced loads / stores is reused, between block barriers, as eight
 // private padded exchange regions (one per wave) for the Stockham stages.
@@ -94,305 +86,6 @@ __device__ __forceinline__ void col_tile(int& plane, int& c0) {
   }
   plane = J / nb;
   c0 = (J - plane * nb) * C::CW;
-}
-
-// ------------------------------------------------------------------ row passes
-// A row workgroup covers rows R0 .. R0 + 4 NB - 1 (R0 = 4 NB blockIdx.x), wave
-// w rows R0 + w NB .. + NB - 1, and its waves' LDS regions hold those rows
-// in order: row R0 + rel at rel * padded(N) (+ the PadLds padding).  In the
-// quad-block layout the same rows are one contiguous run of 4 NB N elements
-// from R0 N, so the workgroup moves them between LDS and memory with
-// consecutive lanes on consecutive elements (whole 128-byte lines).
-static_assert(kWaves == 4, "quad-block row staging assumes 4 waves of rows");
-template <int N>
-__device__ __forceinline__ int rows_stage_addr(int j) {  // LDS slot of element j of the run
-  const int qr = j / (4 * N), rem = j - qr * 4 * N;
-  const int w = rem & 15, rel = 4 * qr + (w >> 2), col = ((rem >> 4) << 2) + (w & 3);
-  return rel * padded(N) + col + (col >> 5);
-}
-template <int N>
-__device__ __forceinline__ int rows_stage_row(int j) {  // row of element j relative to R0
-  const int qr = j / (4 * N), rem = j - qr * 4 * N;
-  return 4 * qr + ((rem & 15) >> 2);
-}
-template <int N>
-__device__ __forceinline__ int rows_stage_col(int j) {
-  const int rem = j % (4 * N);
-  return ((rem >> 4) << 2) + (rem & 3);
-}
-// run (quad-block memory) -> LDS rows; rows at or beyond nrows read as zero
-template <int N, int NB>
-__device__ __forceinline__ void rows_quad_load(float2* lds, const float2* __restrict__ src, int R0, int nrows) {
-  constexpr int TOT = 4 * NB * N, PER = TOT / kThreads;
-  static_assert(PER * kThreads == TOT, "run must divide evenly");
-  float2 t[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int j = threadIdx.x + k * kThreads;
-    t[k] = R0 + rows_stage_row<N>(j) < nrows ? src[(size_t)R0 * N + j] : czero();
-  }
-#pragma unroll
-  for (int k = 0; k < PER; ++k) lds[rows_stage_addr<N>(threadIdx.x + k * kThreads)] = t[k];
-}
-// LDS rows -> run (quad-block memory): dst[j] = f(value, row, col) for rows below nrows
-template <int N, int NB, class Fn>
-__device__ __forceinline__ void rows_quad_store(const float2* lds, float2* __restrict__ dst, int R0, int nrows, Fn&& f) {
-  constexpr int TOT = 4 * NB * N, PER = TOT / kThreads;
-  static_assert(PER * kThreads == TOT, "run must divide evenly");
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int j = threadIdx.x + k * kThreads;
-    const int row = R0 + rows_stage_row<N>(j);
-    if (row < nrows) dst[(size_t)R0 * N + j] = f(lds[rows_stage_addr<N>(j)], row, rows_stage_col<N>(j), (size_t)R0 * N + j);
-  }
-}
-
-// out = (add ? out : 0) + post(scale * F_x(pre * in))   along x, one row per wave
-// (in / out are K when qin / qout: in the quad-block layout, staged through LDS)
-template <int N, bool INV, bool PRE_TAPER, bool POST_TAPER>
-__global__ __launch_bounds__(kThreads) void k_rows(KArgs a) {
-  using C = RowCfg<N>;
-  using F = WaveFft<N, C::NB, false, INV, PadLds<N>>;
-  __shared__ float2 lds[kWaves * C::LDSW];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nrows = a.np * a.NY;
-  const int R0 = blockIdx.x * kWaves * C::NB;
-  const int rb = R0 + wave * C::NB;
-  // K in the quad-block layout goes through LDS as whole lines; row-major K
-  // is read and written like any wavefield
-  const bool qin = a.qin && a.quad, qout = a.qout && a.quad;
-  const bool staged = qin || qout;  // grid-uniform: every wave reaches the barriers
-  if (rb >= nrows && !staged) return;
-  float2* wl = lds + wave * C::LDSW;
-  const float s = a.scale;  // row normalisation 1/sqrt(NX)
-  float2 v[C::V];
-  if (qin) {
-    rows_quad_load<N, C::NB>(lds, a.in, R0, nrows);
-    __syncthreads();
-  }
-  if (rb < nrows) {
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::first(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      float2 x = czero();
-      if (lr < nrows) {
-        x = qin ? wl[PadLds<N>::addr(b, i)] : a.in[(unsigned)(lr * N + i)];
-        if (PRE_TAPER) x = cscale(x, a.tapx[i] * a.tapy[lr % a.NY]);
-      }
-      v[e] = x;
-    }
-    if (qin) wave_sync();  // the transform reuses the region it was read from
-    F::run(v, wl, a.twx, lane);
-  }
-  auto post = [&](float2 y, int lr, int i, unsigned idx) {
-    y = cscale(y, s);
-    if (POST_TAPER) y = cscale(y, a.tapx[i] * a.tapy[lr % a.NY]);
-    if (a.add) y = cadd(y, a.out[idx]);
-    return y;
-  };
-  if (qout) {
-    if (rb < nrows) {
-      wave_sync();
-#pragma unroll
-      for (int e = 0; e < C::V; ++e) {
-        int b, i;
-        edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-        wl[PadLds<N>::addr(b, i)] = v[e];
-      }
-    }
-    __syncthreads();
-    rows_quad_store<N, C::NB>(lds, a.out, R0, nrows, post);
-    return;
-  }
-  if (rb >= nrows) return;
-#pragma unroll
-  for (int e = 0; e < C::V; ++e) {
-    int b, i;
-    edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-    const int lr = rb + b;
-    if (lr < nrows) {
-      const unsigned idx = lr * N + i;
-      a.out[idx] = post(v[e], lr, i, idx);
-    }
-  }
-}
-
-// rows_fanout: W_r = scale * F_x([labels == r] * in) for every reference r
-// (T: arithmetic type of the transforms, float2 or double2)
-template <int N, bool MAP, class T = float2>
-__global__ __launch_bounds__(kThreads) void k_rows_fanout(KArgs a) {
-  using C = RowCfg<N>;
-  using F = WaveFft<N, C::NB, false, false, PadLds<N>, T>;
-  __shared__ T lds[kWaves * C::LDSW];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nrows = a.np * a.NY;
-  const int rb = (blockIdx.x * kWaves + wave) * C::NB;
-  // twiddles in LDS: inside the term loops a global load would wait (one
-  // counter for all vector memory operations) for the term stores / the next
-  // term's loads still in flight
-  __shared__ T twl[N];
-  const T* twg = twx_of(a, (T*)nullptr);
-  for (int i = threadIdx.x; i < N; i += kThreads) twl[i] = twg[i];
-  __syncthreads();
-  if (rb >= nrows) return;
-  T* wl = lds + wave * C::LDSW;
-  T u[C::V];
-  uint8_t lab[C::V];
-#pragma unroll
-  for (int e = 0; e < C::V; ++e) {
-    int b, i;
-    edge_pos<N, C::NB, F::P::first(), false>(lane, e, b, i);
-    const int lr = rb + b;
-    u[e] = cz<T>();
-    lab[e] = 255;
-    if (lr < nrows) {
-      u[e] = from_f2<T>(a.in[(unsigned)(lr * N + i)]);
-      const int p = lr / a.NY, iy = lr - p * a.NY;
-      lab[e] = a.labels[(unsigned)((model_iw<MAP>(a, plane_iw(a, p)) * a.NY + iy) * N + i)];
-    }
-  }
-  const float s = a.scale;
-  uint32_t wm = 0xffffffffu;
-  if (a.rowmask) {
-    wm = 0;
-    for (int b = 0; b < C::NB; ++b) {
-      const int lr = rb + b;
-      if (lr < nrows) {
-        const int p = lr / a.NY;
-        wm |= a.rowmask[model_iw<MAP>(a, plane_iw(a, p)) * a.NY + (lr - p * a.NY)];
-      }
-    }
-    wm = __builtin_amdgcn_readfirstlane(wm);
-  }
-  for (int r = 0; r < a.nref; ++r) {
-    if (r < 32 && !((wm >> r) & 1u)) continue;  // rows without reference r: the column pass reads zeros
-    T x[C::V];
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) x[e] = (lab[e] == r) ? u[e] : cz<T>();
-    F::run(x, wl, twl, lane);
-    float2* W = a.W + (size_t)r * a.wstride;
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      if (lr < nrows) W[widx(a, lr, i, N)] = to_f2(cscale(x[e], s));
-    }
-  }
-}
-
-// rows_select: out = (add ? out : 0) + sum_r [labels == r] * scale * F_x^-1(W_r)
-// KNEXT: also K = scale * F_x(taper * out) (quad-block), the first row pass of
-// a next step that propagates out further: one transform more here instead of
-// a pass that reads out back.
-template <int N, bool MAP, bool KNEXT = false>
-__global__ __launch_bounds__(kThreads) void k_rows_select(KArgs a) {
-  using C = RowCfg<N>;
-  using F = WaveFft<N, C::NB, false, true, PadLds<N>>;
-  using Ff = WaveFft<N, C::NB, false, false, PadLds<N>>;
-  static_assert(F::P::last() == Ff::P::first(), "register hand-off needs mirrored plans");
-  __shared__ float2 lds[kWaves * C::LDSW];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nrows = a.np * a.NY;
-  const int rb = (blockIdx.x * kWaves + wave) * C::NB;
-  // twiddles in LDS: inside the term loops a global load would wait (one
-  // counter for all vector memory operations) for the term stores / the next
-  // term's loads still in flight
-  __shared__ float2 twl[N];
-  for (int i = threadIdx.x; i < N; i += kThreads) twl[i] = a.twx[i];
-  __syncthreads();
-  if (rb >= nrows) return;
-  float2* wl = lds + wave * C::LDSW;
-  uint8_t lab[C::V];
-  float2 acc[C::V];
-#pragma unroll
-  for (int e = 0; e < C::V; ++e) {
-    int b, i;
-    edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-    const int lr = rb + b;
-    acc[e] = czero();
-    lab[e] = 255;
-    if (lr < nrows) {
-      const int p = lr / a.NY, iy = lr - p * a.NY;
-      lab[e] = a.labels[(unsigned)((model_iw<MAP>(a, plane_iw(a, p)) * a.NY + iy) * N + i)];
-    }
-  }
-  // references present in this wave's rows (wave-uniform)
-  uint32_t wm = 0xffffffffu;
-  if (a.rowmask) {
-    wm = 0;
-    for (int b = 0; b < C::NB; ++b) {
-      const int lr = rb + b;
-      if (lr < nrows) {
-        const int p = lr / a.NY;
-        wm |= a.rowmask[model_iw<MAP>(a, plane_iw(a, p)) * a.NY + (lr - p * a.NY)];
-      }
-    }
-    wm = __builtin_amdgcn_readfirstlane(wm);
-  }
-  const uint32_t live = a.nref >= 32 ? wm : (wm & ((1u << a.nref) - 1u));
-  float2 nxt[C::V];
-  auto fetch = [&](int r) {
-    const float2* W = a.W + (size_t)r * a.wstride;
-    // the lane index made opaque here: the per-element offsets are recomputed
-    // per reference (a few integer ops) instead of held in registers
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, F::P::first(), false>(ln, e, b, i);
-      const int lr = rb + b;
-      nxt[e] = lr < nrows ? W[widx(a, lr, i, N)] : czero();
-    }
-  };
-  // absent references contribute nothing to these rows: skip their loads and
-  // transforms.  The next reference's row is fetched into registers during
-  // this one's transform, except at 16 values per lane, where holding it
-  // would cost a wave of occupancy
-  constexpr bool PREFETCH = C::V < 16;
-  int r = a.rowmask ? next_bit(live, -1) : 0;
-  const int rend = a.rowmask ? 32 : a.nref;
-  if (PREFETCH && r < rend) fetch(r);
-  while (r < rend) {
-    if constexpr (!PREFETCH) fetch(r);
-    float2 x[C::V];
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) x[e] = nxt[e];
-    const int rn = a.rowmask ? next_bit(live, r) : r + 1;
-    if (PREFETCH && rn < rend) fetch(rn);
-    F::run(x, wl, twl, lane);
-#pragma unroll
-    for (int e = 0; e < C::V; ++e)
-      if (lab[e] == r) acc[e] = cadd(acc[e], x[e]);
-    r = rn;
-  }
-  const float s = a.scale;
-#pragma unroll
-  for (int e = 0; e < C::V; ++e) {
-    int b, i;
-    edge_pos<N, C::NB, F::P::last(), false>(lane, e, b, i);
-    const int lr = rb + b;
-    if (lr < nrows) {
-      const unsigned idx = lr * N + i;
-      float2 y = cscale(acc[e], s);
-      if (a.add) y = cadd(y, a.out[idx]);
-      if (!KNEXT || a.knext != 2) a.out[idx] = y;
-      if constexpr (KNEXT) acc[e] = cscale(y, a.tapx[i] * a.tapy[lr % a.NY]);
-    }
-  }
-  if constexpr (KNEXT) {
-    Ff::run(acc, wl, twl, lane);
-#pragma unroll
-    for (int e = 0; e < C::V; ++e) {
-      int b, i;
-      edge_pos<N, C::NB, Ff::P::last(), false>(lane, e, b, i);
-      const int lr = rb + b;
-      if (lr < nrows) a.K[widx(a, lr, i, N)] = cscale(acc[e], s);
-    }
-  }
 }
 
 // ------------------------------------------------------------------ column passes
@@ -1145,8 +838,6 @@ __global__ __launch_bounds__(SplitCfg::THREADS) __attribute__((amdgpu_waves_per_
 }
 
 // ------------------------------------------------------------------ launchers
-#define FWIX_SIZES(X) X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(1024)
-
 bool fft_size_supported(int n) {
   switch (n) {
 #define CASE(S) case S:
@@ -1159,121 +850,9 @@ bool fft_size_supported(int n) {
 
 int col_tile_width(int n) { return col_cw(n); }
 
-// Presence masks of reference labels: bit r of rowmask[row] is set when
-// label r occurs in that (w, y) row; planemask is the OR over a plane's rows.
-__global__ __launch_bounds__(kThreads) void k_presence(const uint8_t* __restrict__ labels, uint32_t* rowmask,
-                                                       int NX, long long nrows) {
-  const long long row = (long long)blockIdx.x * kWaves + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= nrows) return;
-  uint32_t m = 0;
-  for (int x = lane; x < NX; x += 64) {
-    const int l = labels[row * NX + x];
-    if (l < 32) m |= 1u << l;
-  }
-  for (int off = 32; off > 0; off >>= 1) m |= (uint32_t)__shfl_xor((int)m, off);
-  if (lane == 0) rowmask[row] = m;
-}
-__global__ __launch_bounds__(kThreads) void k_planemask(const uint32_t* __restrict__ rowmask, uint32_t* planemask,
-                                                        int NY, long long nplanes) {
-  const long long p = (long long)blockIdx.x * kThreads + threadIdx.x;
-  if (p >= nplanes) return;
-  uint32_t m = 0;
-  for (int y = 0; y < NY; ++y) m |= rowmask[p * NY + y];
-  planemask[p] = m;
-}
-// number of present (row, reference) pairs of every plane
-__global__ __launch_bounds__(kThreads) void k_present_count(const uint32_t* __restrict__ rowmask, int* cnt, int NY,
-                                                            long long nplanes, uint32_t refs) {
-  const long long p = (long long)blockIdx.x * kThreads + threadIdx.x;
-  if (p >= nplanes) return;
-  int c = 0;
-  for (int y = 0; y < NY; ++y) c += __builtin_popcount(rowmask[p * NY + y] & refs);
-  cnt[p] = c;
-}
-hipError_t launch_present_count(const uint32_t* rowmask, int* cnt, int NY, long long nplanes, int nref,
-                                hipStream_t st) {
-  const uint32_t refs = nref >= 32 ? 0xffffffffu : ((1u << nref) - 1u);
-  hipLaunchKernelGGL(k_present_count, dim3((unsigned)((nplanes + kThreads - 1) / kThreads)), dim3(kThreads), 0, st,
-                     rowmask, cnt, NY, nplanes, refs);
-  return hipGetLastError();
-}
-
-hipError_t launch_presence(const uint8_t* labels, uint32_t* rowmask, uint32_t* planemask, int NX, int NY,
-                           long long nplanes, hipStream_t st) {
-  const long long nrows = nplanes * NY;
-  hipLaunchKernelGGL(k_presence, dim3((unsigned)((nrows + kWaves - 1) / kWaves)), dim3(kThreads), 0, st, labels,
-                     rowmask, NX, nrows);
-  hipLaunchKernelGGL(k_planemask, dim3((unsigned)((nplanes + kThreads - 1) / kThreads)), dim3(kThreads), 0, st,
-                     rowmask, planemask, NY, nplanes);
-  return hipGetLastError();
-}
-
-template <class Fn>
-static hipError_t dispatch_n(int n, Fn&& fn) {
-  switch (n) {
-#define CASE(S) case S: return fn(std::integral_constant<int, S>{});
-    FWIX_SIZES(CASE)
-#undef CASE
-    default: return hipErrorInvalidValue;
-  }
-}
-
-static dim3 row_grid(int N, int nrows) {
-  const int nb = row_nb(N);
-  const int waves = (nrows + nb - 1) / nb;
-  return dim3((waves + kWaves - 1) / kWaves);
-}
 static dim3 col_grid(int N, int NX, int np) {
   const int cw = col_cw(N);
   return dim3((NX + cw - 1) / cw, np);
-}
-
-// kind: 0 plain forward, 1 plain inverse, 2 forward with pre-taper,
-//       3 inverse with post-taper
-hipError_t launch_rows(int kind, const KArgs& a, hipStream_t st) {
-  return dispatch_n(a.NX, [&](auto nc) -> hipError_t {
-    constexpr int N = decltype(nc)::value;
-    const dim3 g = row_grid(N, a.np * a.NY);
-    switch (kind) {
-      case 0: hipLaunchKernelGGL((k_rows<N, false, false, false>), g, dim3(kThreads), 0, st, a); break;
-      case 1: hipLaunchKernelGGL((k_rows<N, true, false, false>), g, dim3(kThreads), 0, st, a); break;
-      case 2: hipLaunchKernelGGL((k_rows<N, false, true, false>), g, dim3(kThreads), 0, st, a); break;
-      case 3: hipLaunchKernelGGL((k_rows<N, true, false, true>), g, dim3(kThreads), 0, st, a); break;
-      default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-  });
-}
-
-hipError_t launch_rows_fanout(const KArgs& a, hipStream_t st) {
-  return dispatch_n(a.NX, [&](auto nc) -> hipError_t {
-    constexpr int N = decltype(nc)::value;
-    const dim3 g = row_grid(N, a.np * a.NY);
-    if (a.f64) {
-      if (a.mplane) hipLaunchKernelGGL((k_rows_fanout<N, true, double2>), g, dim3(kThreads), 0, st, a);
-      else hipLaunchKernelGGL((k_rows_fanout<N, false, double2>), g, dim3(kThreads), 0, st, a);
-    } else {
-      if (a.mplane) hipLaunchKernelGGL((k_rows_fanout<N, true>), g, dim3(kThreads), 0, st, a);
-      else hipLaunchKernelGGL((k_rows_fanout<N, false>), g, dim3(kThreads), 0, st, a);
-    }
-    return hipGetLastError();
-  });
-}
-
-hipError_t launch_rows_select(const KArgs& a, hipStream_t st) {
-  return dispatch_n(a.NX, [&](auto nc) -> hipError_t {
-    constexpr int N = decltype(nc)::value;
-    const dim3 g = row_grid(N, a.np * a.NY);
-    if (a.knext) {
-      if (a.mplane) hipLaunchKernelGGL((k_rows_select<N, true, true>), g, dim3(kThreads), 0, st, a);
-      else hipLaunchKernelGGL((k_rows_select<N, false, true>), g, dim3(kThreads), 0, st, a);
-    } else {
-      if (a.mplane) hipLaunchKernelGGL((k_rows_select<N, true>), g, dim3(kThreads), 0, st, a);
-      else hipLaunchKernelGGL((k_rows_select<N, false>), g, dim3(kThreads), 0, st, a);
-    }
-    return hipGetLastError();
-  });
 }
 
 hipError_t launch_cols(bool inv, const KArgs& a, hipStream_t st) {

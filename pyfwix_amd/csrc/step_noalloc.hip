@@ -106,7 +106,7 @@ __global__ void k_step_tables(float* kx, float* ky, float* w2, float* tapx, floa
   if (i < NX) {
     kx[i] = kval(i, NX, dx);
     tapx[i] = tap(i, NX, tx);
-    twx[i] = tw(i, NX);
+    twx[i] = tw(twiddle_exp(NX, false, i), NX);
   }
   if (i < NY) {
     ky[i] = kval(i, NY, dy);
