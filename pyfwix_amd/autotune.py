@@ -42,8 +42,8 @@ def set_budget(kind: int, mode: int, n: int, wpe: int) -> None:
 
 
 def get_layout(kind: int, mode: int, n: int) -> int:
-    """Layout of the column transforms for (kind, mode, column length n): 0 one
-    wave per column, 1 two waves per column (n = 1024 only)."""
+    """Layout of the column transforms for (kind, mode, column length n): 0 tiles
+    of 8 columns, 1 tiles of 4 (n = 1024 only)."""
     v = _lib.lib.fwix_tune_columns_layout_get(int(kind), int(mode), int(n))
     if v < 0:
         raise ValueError(f"no column kernel for kind={kind} mode={mode} n={n}")
@@ -106,10 +106,10 @@ def tune_size(n: int, planes: int | None = None, nref: int = 4, taylor: int = 1,
     labels (1, planes, n, n)) device tensors and ``freqs`` (planes values, Hz)
     tune on a real depth of a workload (which references are present in which
     rows changes what the fan-out / fan-in transforms do); by default the
-    labels are random.  At n = 1024 the two-wave layout is timed beside the
-    one-wave one.  Returns {"fanout": {config: us}, "fanin": {...},
+    labels are random.  At n = 1024 the 4-column layout is timed beside the
+    8-column one.  Returns {"fanout": {config: us}, "fanin": {...},
     "scatter_fanout": {...}, "scatter_fanin": {...}, "chosen": {...}}, config
-    "4" for one wave per column at 4 waves per SIMD, "split4" for two."""
+    "4" for layout 0 at 4 waves per SIMD, "split4" for layout 1."""
     import torch
     from .ops import FWIX_PSPI, OneStep, Scatter, make_dims
     dev = torch.device(device or "cuda:0")
@@ -147,8 +147,8 @@ def tune_size(n: int, planes: int | None = None, nref: int = 4, taylor: int = 1,
         scat.forward(False, u, v)
         scat.adjoint(False, w, v)
 
-    # configurations: register budget, and at n = 1024 also the two-wave layout
-    # (keys "4" = one wave per column at 4 waves per SIMD, "split4" = two waves)
+    # configurations: register budget, and at n = 1024 also the 4-column layout
+    # (keys "4" = layout 0 at 4 waves per SIMD, "split4" = layout 1)
     configs = [(0, w) for w in candidates]
     if n == 1024:
         configs += [(1, w) for w in candidates]

@@ -124,11 +124,11 @@ static std::vector<double2> twiddle_table64(int n) {  // exp(-2 pi i k / n) in d
   }
   return t;
 }
-// the row transforms' stage twiddles (twiddle_exp) of the float32 or float64 plan, in double
-static std::vector<double2> stage_twiddles(int n, bool f64) {
+// the stage twiddles (twiddle_exp) of one kind of plan, in double
+static std::vector<double2> stage_twiddles(int n, PlanKind kind) {
   const auto t = twiddle_table64(n);
   std::vector<double2> o(n);
-  for (int i = 0; i < n; ++i) o[i] = t[twiddle_exp(n, f64, i)];
+  for (int i = 0; i < n; ++i) o[i] = t[twiddle_exp(n, kind, i)];
   return o;
 }
 static std::vector<float2> rounded(const std::vector<double2>& t64) {
@@ -136,10 +136,6 @@ static std::vector<float2> rounded(const std::vector<double2>& t64) {
   for (size_t k = 0; k < t.size(); ++k) t[k] = make_float2((float)t64[k].x, (float)t64[k].y);
   return t;
 }
-static std::vector<float2> twiddle_table(int n) {  // the float64 table rounded once
-  return rounded(twiddle_table64(n));
-}
-
 void validate_dims(const fwix_dims* d, bool need_fft) {
   if (!d) throw Error("null dims");
   if (d->NX < 1 || d->NY < 1 || d->NW < 1 || d->NS < 1) throw Error("dims: NX, NY, NW, NS must be >= 1");
@@ -181,10 +177,10 @@ void Tables::init(const fwix_dims& d, int tx, int ty) {
   upload_bytes(b_tapx, tx_.data(), tx_.size() * 4);
   upload_bytes(b_tapy, ty_.data(), ty_.size() * 4);
   if (fft_size_supported(d.NX) && fft_size_supported(d.NY)) {
-    auto twx = rounded(stage_twiddles(d.NX, false)), twy = twiddle_table(d.NY);
+    auto twx = rounded(stage_twiddles(d.NX, kRow32)), twy = rounded(stage_twiddles(d.NY, kCol32));
     upload_bytes(b_twx, twx.data(), twx.size() * 8);
     upload_bytes(b_twy, twy.data(), twy.size() * 8);
-    auto twx64 = stage_twiddles(d.NX, true), twy64 = twiddle_table64(d.NY);
+    auto twx64 = stage_twiddles(d.NX, kRow64), twy64 = stage_twiddles(d.NY, kCol64);
     upload_bytes(b_twx64, twx64.data(), twx64.size() * 16);
     upload_bytes(b_twy64, twy64.data(), twy64.size() * 16);
   }
@@ -258,7 +254,7 @@ int auto_chunk(const fwix_dims& d, int nterm, int requested) {
   // fan-out planes).  Chunks are then balanced so the last one is not a
   // small tail.
   const double per_plane = (double)(1 + nterm) * d.NX * d.NY * 8.0;
-  const int cw = fft_size_supported(d.NY) ? col_tile_width(d.NY) : 16;
+  const int cw = d.NY >= 1024 ? 4 : d.NY >= 512 ? 8 : std::max(8, (d.NY % 3 == 0 ? 6144 : 4096) / d.NY);
   const int blocks_per_plane = (d.NX + cw - 1) / cw;
   const int target = nterm > 4 ? 4096 : 32768;
   int c = (target + blocks_per_plane - 1) / blocks_per_plane;

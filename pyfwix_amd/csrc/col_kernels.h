@@ -1,0 +1,251 @@
+// Column passes of the fused depth steps: the tile of a workgroup and its
+// memory accesses, the spectral multipliers, and the launch geometry (kernels:
+// cols_fanout.hip, cols_fanin.hip; the plain transform: step_kernels.hip).
+//
+// A workgroup transforms CW columns of N points (TileFft), loaded from and
+// stored to memory without a staging tile: a wave's access covers 64 / CW
+// rows of CW consecutive columns.
+//
+// What bounds them: vector instructions and memory about equally.  A fan-out
+// of a 512^2 x 64 plane launch with all four references present runs one forward and
+// four inverse transforms, 203 VALU instructions per point (40 per term: 31 of the
+// transform, the rest the multiplier), VALU 60 % busy, while it moves
+// 0.52 GB (3.6 TB/s); LDS is active 36 % of the time without bank conflicts.
+// The form before staged every tile through LDS on the way in and out (one
+// exchange and a barrier more per term) and computed every position and LDS address
+// per element.  Before -> now, us per launch: fan-out 512^2 x 64 planes 175 ->
+// 143, 384^2 x 200 375 -> 270, 1024^2 x 128 1012 -> 884, 192 x 384 x 26 (complex
+// slowness) 92 -> 50, 96 x 128 x 24 25 -> 15; fan-in 212 -> 180, 572 -> 335, 1237 -> 1044,
+// 121 -> 53, 25 -> 14; float64 768^2 x 6 fan-out 222 -> 134, fan-in 443 -> 272.
+#pragma once
+#include "fwix_kernels.h"
+#include "fwix_launch.h"
+
+#include <type_traits>
+
+namespace fwix {
+
+// Workgroups are handed to the 8 XCDs round-robin by linear id, and each
+// XCD has its own L2.  A column tile reads CW * 8 bytes of every row; with
+// CW = 8 (4) that is a half (quarter) of a 128-byte line, so G = 2 (4)
+// neighbouring tiles share every line they read.  Linear ids L, L + 8, ...
+// run on the same XCD back to back, so they take the G parts: within each
+// group of 8G ids, 8G g + 8h + q gets the logical tile 8G g + G q + h (a
+// trailing partial group keeps the identity).  Logical tile J is column
+// tile J % gridDim.x of plane J / gridDim.x.
+template <class F>
+__device__ __forceinline__ void col_tile(int& plane, int& c0) {
+  const int nb = gridDim.x;
+  const int L = blockIdx.y * nb + blockIdx.x;
+  int J = L;
+  constexpr int G = 128 / (F::CW * 8);
+  if constexpr (G > 1) {
+    const int total = nb * gridDim.y;
+    const int r = L % (8 * G);
+    if (L - r + 8 * G <= total) J = L - r + G * (r % 8) + r / 8;
+  }
+  plane = J / nb;
+  c0 = (J - plane * nb) * F::CW;
+}
+
+// Columns per workgroup: 8 (half a line of memory per row; 16 would take the
+// LDS of a second workgroup), 4 for float64 columns from 512 points on (twice
+// the LDS per value) and for 1024 points in the 4-column layout, the default
+// there: its waves access whole quad blocks and three workgroups fit a CU
+// (1024^2 x 16 planes: fan-out 160 us against 227 with 8 columns, fan-in 210 against
+// 253).
+constexpr int col_cw(int N, bool f64, int layout) { return (f64 && N >= 512) || (N == 1024 && layout == 1) ? 4 : 8; }
+
+// One plane of a wavefield (or of a term buffer) as a buffer resource: the
+// base address sits in scalar registers, an element costs one 32-bit lane
+// offset and a uniform offset.  Offsets at or beyond the plane's size read as
+// zero and drop stores (hardware range check), which replaces the per-element
+// bounds and presence branches: such elements get the offset kOff.
+constexpr unsigned kOff = 0x80000000u;
+__device__ __forceinline__ unsigned plane_bytes(const KArgs& a) { return (unsigned)(a.NX * a.NY) * 8u; }
+struct PlaneBuf {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ PlaneBuf(const float2* base, unsigned bytes)
+      : r(__builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)bytes, 0x00020000)) {}
+  __device__ __forceinline__ float2 load(unsigned off, int soff) const {
+    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, soff, 0));
+  }
+  __device__ __forceinline__ void store(float2 v, unsigned off, int soff) const {
+    using U2 = __attribute__((ext_vector_type(2))) unsigned;
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), r, (int)off, soff, 0);
+  }
+};
+// Byte offsets of this thread's elements: its column at rows row + C, C the
+// first (FIRST: row l0) or last positions of the transform, in a row-major
+// plane or (quad) one in the quad-block layout.  When every C is a multiple of
+// 4, C rows move the offset by C NX elements in both layouts; the short columns where
+// one is not (8, 12 and 24 points) form the offset per element.
+template <class F, bool FIRST>
+struct ColOffs {
+  static constexpr int C(int e) { return FIRST ? F::first_c(e) : F::last_c(e); }
+  static constexpr bool by4() {
+    for (int e = 0; e < F::V; ++e)
+      if (C(e) % 4) return false;
+    return true;
+  }
+  unsigned o;
+  int row, col, NX, step;
+  bool quad;
+  __device__ __forceinline__ ColOffs(const F& f, int c0, int NX_, bool quad_)
+      : row(FIRST ? f.l0 : f.lane), col(c0 + f.col), NX(NX_), step(NX_ * 8), quad(quad_) {
+    o = col >= NX ? kOff : (quad ? qidx(row, col, NX) : (unsigned)(row * NX + col)) * 8u;
+  }
+  __device__ __forceinline__ unsigned voff(int e) const {
+    if constexpr (by4()) return o;
+    if (col >= NX) return kOff;
+    return (quad ? qidx(row + C(e), col, NX) : (unsigned)((row + C(e)) * NX + col)) * 8u;
+  }
+  __device__ __forceinline__ int soff(int e) const { return by4() ? C(e) * step : 0; }
+};
+
+// this workgroup's copy of the column transforms' twiddle table and of the
+// plane's row masks (all set when masks are off); the caller synchronises.
+// In LDS because one wait counter covers vector loads and stores: a global
+// load in the loop over the terms would wait for the term's stores or for the
+// next term's tile in flight.
+template <class F, class T>
+__device__ __forceinline__ void col_twiddles(T* twl, const T* __restrict__ tw) {
+  for (int i = threadIdx.x; i < F::TW; i += F::THREADS) twl[i] = tw[i];
+}
+template <class F, int N>
+__device__ __forceinline__ void col_row_masks(uint32_t* rml, const uint32_t* __restrict__ rm) {
+  for (int i = threadIdx.x; i < N; i += F::THREADS) rml[i] = rm ? rm[i] : 0xffffffffu;
+}
+// Reference slowness r of the plane, by a scalar load (through a
+// constant-address-space pointer): that load waits on the scalar counter
+// only, and every workgroup of the plane reads the same few values.
+__device__ __forceinline__ float2 term_sref(const KArgs& a, int r, int iw) {
+  using CP = const __attribute__((address_space(4))) float*;
+  const CP p = (CP)(const void*)a.sref + 2 * (r * a.NW + iw);
+  return make_float2(p[0], p[1]);
+}
+
+// ------------------------------------------------------------------ multipliers
+// Pointwise spectral multiplier of term r at (kx, ky) of frequency iw.
+// MULT 0 / 1: forward / adjoint phase shift of reference slowness r
+// (propagator/src/phase_shift.cu); MULT 2: Born scattering wavenumber factor
+// (|k|/w)^(2it) = (k^2/w^2)^it of Taylor order it = r + 1 (scatter.cu:23-59);
+// order 0 is the identity and is applied in space by the row kernels.
+// The term's uniform part (reference slowness, real/complex branch) is set up
+// once per (plane, term) so the unrolled per-sample loops carry no divergent
+// or if-converted paths.
+template <int MULT, class T>
+struct TermMult {
+  using S = real_of<T>;
+  S w2, wsre, b, iw2, dz;
+  int r;
+  bool real;
+  __device__ __forceinline__ TermMult(const KArgs& a, int r_, int iw, S w2_) : w2(w2_), r(r_), dz(a.dz) {
+    if constexpr (MULT == 2) {
+      iw2 = (S)1 / w2;
+      real = true; wsre = 0; b = 0;
+    } else {
+      const float2 sr = term_sref(a, r_, iw);
+      wsre = w2 * (S)sr.x;
+      b = w2 * ((S)sr.y - (S)a.eps * (S)sr.x);
+      real = b == 0;
+      iw2 = 0;
+    }
+  }
+  // x times the multiplier at k2
+  template <bool REAL>
+  __device__ __forceinline__ T apply(T x, S k2) const {
+    if constexpr (MULT == 2) {
+      const S q = sizeof(S) == 8 ? k2 / w2 : k2 * iw2;
+      S m = q;
+      for (int i = 0; i < r; ++i) m *= q;
+      return cscale(x, m);
+    } else if constexpr (sizeof(S) == 8) {
+      if constexpr (!REAL) return cmul(x, ps_general64<MULT>(wsre - k2, b, dz));
+      else return cmul(x, ps_real64<MULT>(wsre - k2, dz));
+    } else if constexpr (!REAL) {
+      return cmul(x, ps_general<MULT>(wsre - k2, b, dz));
+    } else {
+      // Past the evanescent boundary the multiplier is real and needs no sine
+      // or cosine.  A wave's samples are neighbours in (kx, ky), so most
+      // waves lie on one side (the propagating disc of a 10-20 m grid covers
+      // 3-15 % of the plane): one test of the wave skips both.
+      const float a = wsre - k2, t = __builtin_amdgcn_sqrtf(fabsf(a)) * dz;
+      const float e = __expf(-t);
+      if (__builtin_amdgcn_ballot_w64(a >= 0.f) == 0) return cscale(x, e);
+      float sn, cs;
+      fast_sincos(t, &sn, &cs);
+      const float2 m = a >= 0.f ? make_float2(cs, MULT == 0 ? -sn : sn) : make_float2(e, 0.f);
+      return cmul(x, m);
+    }
+  }
+};
+// k^2 = kx^2 + ky^2 at this thread's samples after a forward transform
+// (the positions of the last stage); loop-invariant over the terms.
+template <class F, class S>
+__device__ __forceinline__ void column_k2(S* k2v, const F& f, const KArgs& a, int c0) {
+  const int col = c0 + f.col;
+  const S kxv = a.kx[col < a.NX ? col : 0];
+  const float* ky = a.ky + f.lane;
+#pragma unroll
+  for (int e = 0; e < F::V; ++e) {
+    const S kyv = ky[F::last_c(e)];
+    if constexpr (sizeof(S) == 8) k2v[e] = fma(kxv, kxv, kyv * kyv);
+    else k2v[e] = fmaf(kxv, kxv, kyv * kyv);
+  }
+}
+
+// ------------------------------------------------------------------ launch geometry
+template <class F>
+inline dim3 col_grid(const KArgs& a) {
+  return dim3((a.NX + F::CW - 1) / F::CW, a.np);
+}
+template <class Fn>
+hipError_t dispatch_wpe(int wpe, Fn&& fn) {
+  switch (wpe) {
+    case 2: return fn(std::integral_constant<int, 2>{});
+    case 4: return fn(std::integral_constant<int, 4>{});
+    case 6: return fn(std::integral_constant<int, 6>{});
+    default: return hipErrorInvalidValue;
+  }
+}
+// mode 0..2 as a constant
+template <class Fn>
+hipError_t dispatch_mode(int mode, Fn&& fn) {
+  switch (mode) {
+    case 0: return fn(std::integral_constant<int, 0>{});
+    case 1: return fn(std::integral_constant<int, 1>{});
+    case 2: return fn(std::integral_constant<int, 2>{});
+    default: return hipErrorInvalidValue;
+  }
+}
+// One column kernel per (size, mode) and, in float32, register budget (2, 4
+// or 6 waves per SIMD, col_wpe_get) and at 1024 points tile width
+// (col_layout_get); float64 arithmetic (a.f64) has one budget.
+// K<N, MODE, WPE, T, CW>::kernel
+template <template <int, int, int, class, int> class K>
+hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) {
+  return dispatch_n(a.NY, [&](auto nc) {
+    constexpr int N = decltype(nc)::value;
+    return dispatch_mode(mode, [&](auto mc) {
+      constexpr int M = decltype(mc)::value;
+      auto go = [&](auto wc, auto cc, auto t) -> hipError_t {
+        using T = decltype(t);
+        constexpr int CW = decltype(cc)::value;
+        using F = TileFft<N, T, CW>;
+        hipLaunchKernelGGL((K<N, M, decltype(wc)::value, T, CW>::kernel), col_grid<F>(a), dim3(F::THREADS), 0, st, a);
+        return hipGetLastError();
+      };
+      constexpr std::integral_constant<int, col_cw(N, true, 0)> cw64{};
+      if (a.f64) return go(std::integral_constant<int, 2>{}, cw64, double2{});
+      return dispatch_wpe(col_wpe_get(kind, mode, N), [&](auto wc) {
+        if constexpr (N == 1024) {
+          if (col_layout_get(kind, mode, N) == 1) return go(wc, std::integral_constant<int, col_cw(N, false, 1)>{}, float2{});
+        }
+        return go(wc, std::integral_constant<int, col_cw(N, false, 0)>{}, float2{});
+      });
+    });
+  });
+}
+
+}  // namespace fwix

@@ -1,22 +1,10 @@
-// Wave-level Stockham FFT for gfx950 (CDNA4, 64-lane wavefronts).
+// FFTs of lines held in registers for gfx950 (CDNA4, 64-lane wavefronts).
 //
-// One wavefront transforms NB batches of N points held as V = NB*N/64 complex
-// values per lane.  The radix plan (8, 4, 3, 2) is fixed at compile time from
-// N and V so every loop unrolls and every index is a constant-folded shift or
-// multiply.  Stages exchange data through the wave's own LDS region and only
-// need wave-level ordering, never a workgroup barrier.
-//
-// Position conventions (Stockham autosort, decimation in time):
-//   stage radix R, sub-transform size Ns (product of earlier radices):
-//     butterfly (b, j), j < N/R, reads  x[b][j + r*N/R]
-//     writes y[b][(j/Ns)*Ns*R + j%Ns + r*Ns]
-//   The first stage therefore reads positions j + r*N/R0 and the last stage
-//   writes positions j + r*N/RL, both contiguous across lanes: kernels load
-//   the first stage straight from global memory and store the last stage
-//   straight back.  The inverse plan is the forward plan reversed, so the
-//   inverse's first stage reads exactly the positions the forward's last
-//   stage wrote: a forward -> pointwise multiply -> inverse chain never leaves
-//   registers between the two transforms.
+// L = N / V lanes hold one line of N points, V complex values each, with the
+// radix plan fixed at compile time.  Stages exchange data through LDS.  Two
+// owners of a line: LaneFft, a line inside one wave (the row passes), and
+// TileFft, the columns of a tile across the waves of a workgroup (the column
+// passes).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -72,45 +60,6 @@ template <bool INV, class T>
 __device__ __forceinline__ T mul_si(T a) {
   return INV ? CX<T>::mk(-a.y, a.x) : CX<T>::mk(a.y, -a.x);
 }
-
-// ----------------------------------------------------------------- compile-time plan
-constexpr int kRadices[4] = {8, 4, 3, 2};
-
-constexpr int plan_len(int N, int V) {
-  int n = N, c = 0;
-  for (int k = 0; k < 4; ++k) {
-    const int R = kRadices[k];
-    while (n % R == 0 && V % R == 0) { n /= R; ++c; }
-  }
-  return n == 1 ? c : -1;
-}
-
-constexpr int plan_radix(int N, int V, int s) {
-  int n = N, c = 0;
-  for (int k = 0; k < 4; ++k) {
-    const int R = kRadices[k];
-    while (n % R == 0 && V % R == 0) {
-      if (c == s) return R;
-      n /= R; ++c;
-    }
-  }
-  return 0;
-}
-
-// radix of stage s of the forward (INV=false) or inverse (reversed) plan
-template <int N, int V, bool INV>
-struct Plan {
-  static constexpr int S = plan_len(N, V);
-  static_assert(S > 0, "FFT size has no radix plan for this register budget");
-  static constexpr int radix(int s) { return plan_radix(N, V, INV ? (S - 1 - s) : s); }
-  static constexpr int ns(int s) {  // product of the radices of stages < s
-    int p = 1;
-    for (int k = 0; k < s; ++k) p *= radix(k);
-    return p;
-  }
-  static constexpr int first() { return radix(0); }
-  static constexpr int last() { return radix(S - 1); }
-};
 
 // ----------------------------------------------------------------- in-register DFTs
 template <int R, bool INV> struct Dft;
@@ -237,116 +186,10 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// ----------------------------------------------------------------- positions
-// Butterfly t = lane + 64*q of a radix-R stage owns batch b and index j.
-// BFAST: batch index varies fastest across lanes (column tiles), else the
-// position within the batch does (rows).
-// (Unsigned arithmetic: t is never negative, and the lane index is opaque to
-// the compiler inside a transform, so signed division would cost sign fix-ups.)
-template <int N, int NB, int R, bool BFAST>
-__device__ __forceinline__ void bj(int t, int& b, int& j) {
-  const unsigned u = (unsigned)t;
-  if (BFAST) { b = (int)(u % NB); j = (int)(u / NB); }
-  else { b = (int)(u / (N / R)); j = (int)(u % (N / R)); }
-}
-
-// (batch, position) of value v = q*R + r at the input of a stage of radix R
-// when it is the first stage, or at the output when it is the last stage.
-template <int N, int NB, int R, bool BFAST>
-__device__ __forceinline__ void edge_pos(int lane, int v, int& b, int& i) {
-  const int q = v / R, r = v % R;
-  int j;
-  bj<N, NB, R, BFAST>(lane + 64 * q, b, j);
-  i = j + r * (N / R);
-}
-
-// ----------------------------------------------------------------- the transform
-// LDS layout policy: L::addr(b, i) gives the element offset of batch b, point i
-// inside the wave's region.  T is the arithmetic type of the values, the LDS
-// region and the twiddle table (float2, or double2 for float64 arithmetic).
-template <int N, int NB, bool BFAST, bool INV, class L, class T = float2>
-struct WaveFft {
-  static constexpr int V = NB * N / 64;
-  using P = Plan<N, V, INV>;
-  static constexpr int S = P::S;
-
-  template <int R, int Ns>
-  __device__ __forceinline__ static void butterflies(T* v, const T* __restrict__ tw, int lane) {
-#pragma unroll
-    for (int q = 0; q < V / R; ++q) {
-      T* x = v + q * R;
-      if constexpr (Ns > 1) {
-        int b, j;
-        bj<N, NB, R, BFAST>(lane + 64 * q, b, j);
-        const int k = (int)((unsigned)j % Ns);
-        constexpr int step = N / (Ns * R);
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-          T w = tw[r * k * step];
-          if (INV) w.y = -w.y;
-          x[r] = cmul(x[r], w);
-        }
-      }
-      Dft<R, INV>::run(x);
-    }
-  }
-
-  template <int R, int Ns, int R2>
-  __device__ __forceinline__ static void exchange(T* v, T* lds, int lane) {
-#pragma unroll
-    for (int q = 0; q < V / R; ++q) {
-      int b, j;
-      bj<N, NB, R, BFAST>(lane + 64 * q, b, j);
-      const unsigned uj = (unsigned)j;
-      const int base = (int)((uj / Ns) * Ns * R + (uj % Ns));
-#pragma unroll
-      for (int r = 0; r < R; ++r) lds[L::addr(b, base + r * Ns)] = v[q * R + r];
-    }
-    wave_sync();
-#pragma unroll
-    for (int q = 0; q < V / R2; ++q) {
-      int b, j;
-      bj<N, NB, R2, BFAST>(lane + 64 * q, b, j);
-#pragma unroll
-      for (int r = 0; r < R2; ++r) v[q * R2 + r] = lds[L::addr(b, j + r * (N / R2))];
-    }
-    wave_sync();
-  }
-
-  template <int s>
-  __device__ __forceinline__ static void stages(T* v, T* lds, const T* __restrict__ tw, int lane) {
-    if constexpr (s < S) {
-      constexpr int R = P::radix(s);
-      constexpr int Ns = P::ns(s);
-      butterflies<R, Ns>(v, tw, lane);
-      if constexpr (s + 1 < S) {
-        exchange<R, Ns, P::radix(s + 1)>(v, lds, lane);
-        stages<s + 1>(v, lds, tw, lane);
-      }
-    }
-  }
-
-  // v holds the values at first-stage input positions (edge_pos<..., P::first()>);
-  // on return it holds the spectrum at last-stage output positions
-  // (edge_pos<..., P::last()>).  Unnormalized.
-  __device__ __forceinline__ static void run(T* v, T* lds, const T* __restrict__ tw, int lane) {
-    // Keep the twiddles and the per-element twiddle / LDS addresses next to
-    // their use: without these fences the compiler hoists every stage's
-    // (loop-invariant) loads and addresses out of the per-reference loops
-    // of the fused kernels and runs out of registers.  The lane index is
-    // made opaque here, so the index arithmetic derived from it is redone
-    // per transform (a few integer ops) instead of held in registers.
-    asm volatile("" ::: "memory");
-    asm volatile("" : "+v"(lane));
-    stages<0>(v, lds, tw, lane);
-  }
-};
-
-// ================================================================= lane transform
-// The transforms of the row passes.  L = N / V lanes hold one line of N
-// points, V values each, and a wave holds 64 / L lines; lane l of a line owns
-// the butterflies j = l + L q of every stage.  The plans below take few,
-// wide stages (their count is what sets the LDS exchanges), with V a multiple
+// ================================================================= stages
+// L = N / V lanes hold one line of N points; lane l of a line owns the
+// butterflies j = l + L q of every stage.  The plans below take few, wide
+// stages (their count is what sets the LDS exchanges), with V a multiple
 // of every radix and L a divisor (or a multiple) of every sub-transform
 // length, so that every position, LDS address and twiddle index of a value is
 // a per-lane base plus a compile-time constant: the loops carry no index
@@ -359,16 +202,25 @@ struct WaveFft {
 //   inverse: the forward stages undone in reverse order (butterfly, then the
 //     conjugate twiddles, exchanges written where the forward reads and read
 //     where it writes), so it starts at the positions the forward ends at and
-//     ends where the forward starts.
+//     ends where the forward starts: a forward -> pointwise multiply -> inverse
+//     chain never leaves registers between the two transforms.
 struct PlanDef {
   int V, S, R[4];
 };
-// Short lines take narrow plans (V <= 12): their launches are small and more
+// Row plans and column plans, float32 and float64 arithmetic.
+enum PlanKind { kRow32 = 0, kRow64 = 1, kCol32 = 2, kCol64 = 3 };
+// Rows: short lines take narrow plans (V <= 12): their launches are small and more
 // waves in flight are worth more than a stage less (256 points: Born adjoint
 // rows 21.3 us at V = 16, two stages, 17.5 us at V = 8, three).  The long
 // lines with a factor 3 take V = 24 (768 points: 4 stages of V = 12 against 3);
 // float64 lines hold at most 16 values per lane (twice the registers each).
-__host__ __device__ constexpr PlanDef plan_def(int N, bool f64) {
+// Columns: a first radix R(0) that divides the lanes a wave holds of a column
+// (TileFft), and V <= 12 below 1024 points: these kernels hold two or three
+// arrays of V values per lane (V = 24 at 384 / 768 points, one stage less:
+// fan-out 193 against 180 us / 194 against 198 us, fan-in 233 against 211 us / 262 against
+// 282 us, Taylor-term fan-out 68 against 57 us / 80 against 67 us, 16 M points).
+__host__ __device__ constexpr PlanDef plan_def(int N, PlanKind kind) {
+  const bool f64 = kind == kRow64 || kind == kCol64, col = kind >= kCol32;
   switch (N) {
     case 8: return {4, 2, {4, 2}};
     case 12: return {12, 1, {12}};
@@ -381,10 +233,12 @@ __host__ __device__ constexpr PlanDef plan_def(int N, bool f64) {
     case 128: return {8, 3, {8, 4, 4}};
     case 192: return {12, 3, {4, 4, 12}};
     case 256: return {8, 3, {8, 8, 4}};
-    case 384: return f64 ? PlanDef{12, 4, {4, 4, 4, 6}} : PlanDef{24, 3, {8, 8, 6}};
+    case 384: return f64 || col ? PlanDef{12, 4, {4, 4, 4, 6}} : PlanDef{24, 3, {8, 8, 6}};
     case 512: return {8, 3, {8, 8, 8}};
-    case 768: return f64 ? PlanDef{12, 4, {4, 4, 4, 12}} : PlanDef{24, 3, {8, 8, 12}};
-    case 1024: return {16, 3, {16, 8, 8}};
+    case 768: return f64 || col ? PlanDef{12, 4, {4, 4, 4, 12}} : PlanDef{24, 3, {8, 8, 12}};
+    case 1024:
+      if (kind == kCol64) return {8, 4, {4, 4, 8, 8}};
+      return col ? PlanDef{16, 3, {4, 16, 16}} : PlanDef{16, 3, {16, 8, 8}};
     default: return {0, 0, {}};
   }
 }
@@ -397,8 +251,8 @@ __host__ __device__ constexpr int plan_ns(const PlanDef& d, int s) {
 // Stage s holds its R - 1 rows of Ns factors one after another ([r][k], k
 // fastest), so a lane reads W^(rk) at a base of its own plus r Ns, neighbouring
 // lanes on neighbouring entries.  Entries past the last stage's are zero.
-__host__ __device__ constexpr int twiddle_exp(int N, bool f64, int i) {
-  const PlanDef d = plan_def(N, f64);
+__host__ __device__ constexpr int twiddle_exp(int N, PlanKind kind, int i) {
+  const PlanDef d = plan_def(N, kind);
   int o = 0;
   for (int s = 1; s < d.S; ++s) {
     const int Ns = plan_ns(d, s), n = (d.R[s] - 1) * Ns;
@@ -411,21 +265,62 @@ __host__ __device__ constexpr int twiddle_exp(int N, bool f64, int i) {
   return 0;
 }
 
-template <int N, class T = float2>
-struct LaneFft {
+// the plan of a line, its positions, twiddles and butterflies
+template <int N, class T, bool COL>
+struct Stages {
   // (a constexpr array member would be a device constant, loaded at run time:
   // the plan is only ever read through these functions)
-  static constexpr bool F64 = sizeof(T) == 16;
-  static constexpr int V = plan_def(N, F64).V, S = plan_def(N, F64).S, L = N / V, NB = 64 / L;
-  static_assert(V > 0 && L * V == N && NB * L == 64, "lanes must divide the line and the wave");
-  static constexpr int R(int s) { return plan_def(N, F64).R[s]; }
-  static constexpr int Ns(int s) { return plan_ns(plan_def(N, F64), s); }
+  static constexpr PlanKind KIND = COL ? (sizeof(T) == 16 ? kCol64 : kCol32) : (sizeof(T) == 16 ? kRow64 : kRow32);
+  static constexpr int V = plan_def(N, KIND).V, S = plan_def(N, KIND).S, L = N / V;
+  static_assert(V > 0 && L * V == N, "lanes must divide the line");
+  static constexpr int R(int s) { return plan_def(N, KIND).R[s]; }
+  static constexpr int Ns(int s) { return plan_ns(plan_def(N, KIND), s); }
   static constexpr int tw_off(int s) {
     int o = 0;
     for (int k = 1; k < s; ++k) o += (R(k) - 1) * Ns(k);
     return o;
   }
   static constexpr int TW = tw_off(S) > 0 ? tw_off(S) : 1;  // table entries (N - R(0))
+
+  // position of value v of lane l before the first forward stage (= after the
+  // inverse) and after the last (= before the inverse): lane base + constant
+  static constexpr int in_c(int s, int v) { return L * (v / R(s)) + (v % R(s)) * (N / R(s)); }
+  static constexpr int first_c(int v) { return in_c(0, v); }
+  static constexpr int last_c(int v) { return in_c(S - 1, v); }
+
+  template <int s, bool INV>
+  __device__ __forceinline__ static void twiddle(T* v, const T* __restrict__ tw, int l) {
+    if constexpr (s > 0) {
+      constexpr int n = Ns(s);
+      static_assert(L % n == 0 || n % L == 0, "a lane's twiddles must sit at constant offsets");
+      const T* t = tw + tw_off(s) + (L % n == 0 ? (int)((unsigned)l % (unsigned)n) : l);
+#pragma unroll
+      for (int q = 0; q < V / R(s); ++q) {
+        const int kc = L % n == 0 ? 0 : (L * q) % n;
+#pragma unroll
+        for (int r = 1; r < R(s); ++r) {
+          const T w = t[(r - 1) * n + kc];
+          T& x = v[q * R(s) + r];
+          x = INV ? cmulc(x, w) : cmul(x, w);
+        }
+      }
+    }
+  }
+  template <int s, bool INV>
+  __device__ __forceinline__ static void butterflies(T* v) {
+#pragma unroll
+    for (int q = 0; q < V / R(s); ++q) Dft<R(s), INV>::run(v + q * R(s));
+  }
+};
+
+// ================================================================= lines of one wave
+// A wave holds NB = 64 / L lines, each on its own L lanes.
+template <int N, class T = float2>
+struct LaneFft : Stages<N, T, false> {
+  using B = Stages<N, T, false>;
+  using B::L; using B::S; using B::V; using B::R; using B::Ns; using B::in_c;
+  static constexpr int NB = 64 / L;
+  static_assert(NB * L == 64, "lanes must divide the wave");
 
   // Padding of the exchange between stages s and s + 1, in positions: Ns more
   // after each block of G, but none where the sum reaches a row of banks (32).
@@ -453,12 +348,6 @@ struct LaneFft {
   // 32); the others 8 past a multiple of 32, so that four rows staged as
   // quads fall into distinct banks
   static constexpr int STRIDE = stride_min() + ((L < 32 ? L : 8) + 32 * 64 - stride_min() % 32) % 32;
-
-  // position of value v of lane l before the first forward stage (= after the
-  // inverse) and after the last (= before the inverse): lane base + constant
-  static constexpr int in_c(int s, int v) { return L * (v / R(s)) + (v % R(s)) * (N / R(s)); }
-  static constexpr int first_c(int v) { return in_c(0, v); }
-  static constexpr int last_c(int v) { return in_c(S - 1, v); }
 
   // exchange after stage s: LDS offset of value v where stage s + 1 reads
   // (IN) and where stage s wrote (OUT), as a lane base and a constant
@@ -508,29 +397,6 @@ struct LaneFft {
     return true;
   }
 
-  template <int s, bool INV>
-  __device__ __forceinline__ static void twiddle(T* v, const T* __restrict__ tw, int l) {
-    if constexpr (s > 0) {
-      constexpr int n = Ns(s);
-      static_assert(L % n == 0 || n % L == 0, "a lane's twiddles must sit at constant offsets");
-      const T* t = tw + tw_off(s) + (L % n == 0 ? (int)((unsigned)l % (unsigned)n) : l);
-#pragma unroll
-      for (int q = 0; q < V / R(s); ++q) {
-        const int kc = L % n == 0 ? 0 : (L * q) % n;
-#pragma unroll
-        for (int r = 1; r < R(s); ++r) {
-          const T w = t[(r - 1) * n + kc];
-          T& x = v[q * R(s) + r];
-          x = INV ? cmulc(x, w) : cmul(x, w);
-        }
-      }
-    }
-  }
-  template <int s, bool INV>
-  __device__ __forceinline__ static void butterflies(T* v) {
-#pragma unroll
-    for (int q = 0; q < V / R(s); ++q) Dft<R(s), INV>::run(v + q * R(s));
-  }
   template <int s>
   __device__ __forceinline__ static void put_out(const T* v, T* line, int l) {
     static_assert(out_ok<s>(), "exchange positions must split into lane base and constant");
@@ -563,8 +429,8 @@ struct LaneFft {
   template <int FROM, int TO>
   __device__ __forceinline__ static void forward(T* v, T* line, const T* __restrict__ tw, int l) {
     if constexpr (FROM < TO) {
-      twiddle<FROM, false>(v, tw, l);
-      butterflies<FROM, false>(v);
+      B::template twiddle<FROM, false>(v, tw, l);
+      B::template butterflies<FROM, false>(v);
       if constexpr (FROM + 1 < TO) {
         put_out<FROM>(v, line, l);
         wave_sync();
@@ -578,8 +444,8 @@ struct LaneFft {
   template <int FROM, int TO>
   __device__ __forceinline__ static void inverse(T* v, T* line, const T* __restrict__ tw, int l) {
     if constexpr (FROM > TO) {
-      butterflies<FROM - 1, true>(v);
-      twiddle<FROM - 1, true>(v, tw, l);
+      B::template butterflies<FROM - 1, true>(v);
+      B::template twiddle<FROM - 1, true>(v, tw, l);
       if constexpr (FROM - 1 > TO) {
         put_in<FROM - 2>(v, line, l);
         wave_sync();
@@ -598,6 +464,163 @@ struct LaneFft {
     asm volatile("" ::: "memory");
     if constexpr (INV) inverse<S, 0>(v, line, tw, l);
     else forward<0, S>(v, line, tw, l);
+  }
+};
+
+// ================================================================= columns of a workgroup
+// A tile of CW columns of N points on CW L threads: thread t holds column
+// t % CW at lane t / CW, V values.  Values are loaded from and stored to
+// memory straight at the positions the first stage reads (a wave's access
+// touches 64 / CW rows of 8 CW bytes) or the last stage writes; no staging
+// tile.  LDS is only the exchange region, in slots of CW values, and a wave
+// holds LW = 64 / CW lanes of every column.
+//
+// Exchange 0 stays inside the waves: position p of it belongs to the wave
+// (p % L) / LW that reads it for stage 1 (lane p % L), and the first stage's
+// lanes are dealt out so that the same wave has written it: lane
+//   l0 = (i / D) (L / R(0)) + D w + i % D,   D = LW / R(0)
+// for place i of wave w.  Each wave's positions form a section of SEC slots;
+// exchange 1 keeps a wave's output positions of stage 1 in its own section
+// too.  So a forward transform waits for the workgroup before its first
+// write (the exchange before may still be read) and once in exchange 1, an
+// inverse before and in exchange 1, and nothing else (a fourth stage adds one
+// exchange over the whole region, two waits).
+// Tiles of one wave (short columns) need no wait at all.
+template <int N, class T, int CWX>
+struct TileFft : Stages<N, T, true> {
+  using B = Stages<N, T, true>;
+  using B::L; using B::S; using B::V; using B::R; using B::Ns; using B::in_c;
+  static constexpr int CW = CWX * L >= 64 ? CWX : 64 / L;
+  static constexpr int THREADS = CW * L, WAVES = THREADS / 64, LW = 64 / CW;
+  static constexpr bool ONE = WAVES == 1;
+  static constexpr bool SECT = S > 1 && LW % R(0) == 0;
+  static constexpr int D = SECT ? LW / R(0) : 1;
+  static constexpr int ROWL = LW + D, SEC = V * ROWL;  // a section: V rows of LW positions, padded
+  static_assert(THREADS % 64 == 0 && LW * CW == 64, "a wave must hold whole lanes of the tile");
+  static_assert(ONE || S < 3 || SECT, "the first radix must divide a wave's lanes");
+  // slots of the region: the sections, or (one wave, first radix above its
+  // lanes) the positions with one more slot per first-stage butterfly
+  static constexpr int SLOTS = S == 1 ? 1 : SECT ? WAVES * SEC : N + N / R(0);
+  static constexpr int SMEM = SLOTS * CW;
+  // Slot of position p of the exchange after stage s.  Padding: 32 (16 for
+  // float64) lanes of an access sit on 32 / CW places, which must fall into
+  // distinct rows of banks; written places of exchange 0 are a row of the
+  // section or R(0) positions apart, of exchange 1 Ns R(1) positions apart
+  // at each Ns-th.
+  template <int s>
+  __host__ __device__ static constexpr int slot(int pos) {
+    const unsigned p = (unsigned)pos;
+    constexpr unsigned r0 = R(0);
+    if constexpr (s == 0) {
+      if constexpr (!SECT) return (int)(p + p / r0);
+      const unsigned w = p % L / LW, m = p / L, x = p % LW;
+      return (int)(w * SEC + m * ROWL + x + (D > 1 ? x / r0 : 0u));
+    } else if constexpr (s == 1 && !ONE) {
+      constexpr unsigned blk = LW * R(1), grp = Ns(1) * R(1), pad = Ns(1) < 32 / CW ? Ns(1) : 0;
+      static_assert((int)(blk + pad * (blk / grp)) * (V / R(1)) <= SEC, "a wave's stage-1 outputs must fit its section");
+      const unsigned b = p / blk, x = p % blk;
+      return (int)(b % WAVES * SEC + b / WAVES * (blk + pad * (blk / grp)) + x + x / grp * pad);
+    } else {
+      return pos;
+    }
+  }
+  // the positions of value v of lane l after stage s (written by the
+  // forward), and before stage s + 1 (read): lane part and constant part
+  template <int s> __host__ __device__ static constexpr int out_l(int l) {
+    constexpr unsigned n = Ns(s), r = R(s);
+    return (int)((unsigned)l / n * n * r + (unsigned)l % n);
+  }
+  template <int s> static constexpr int out_v(int v) {
+    constexpr int n = Ns(s), r = R(s);
+    return v / r * L * r + v % r * n;
+  }
+  template <int s> static constexpr int in_v(int v) {
+    constexpr int r = R(s + 1);
+    return v / r * L + v % r * (N / r);
+  }
+  __host__ __device__ static constexpr int lane0(int lane) {
+    if constexpr (S == 1 || !SECT) return lane;
+    constexpr unsigned r0 = R(0);
+    const unsigned w = (unsigned)lane / LW, i = (unsigned)lane % LW;
+    return (int)(i / D * (L / r0) + D * w + i % D);
+  }
+  // slots split into lane part and constant, and exchanges 0 and 1 stay in
+  // the sections they must
+  template <int s>
+  static constexpr bool slots_ok() {
+    if (s > 1 || (s == 1 && ONE)) return true;  // a slot is its position
+    int so[V] = {}, si[V] = {};
+    for (int v = 0; v < V; ++v) so[v] = slot<s>(out_v<s>(v)), si[v] = slot<s>(in_v<s>(v));
+    for (int l = 0; l < L; ++l) {
+      const int ol = out_l<s>(s == 0 ? lane0(l) : l), lo = slot<s>(ol), li = slot<s>(l);
+      for (int v = 0; v < V; ++v) {
+        const int o = slot<s>(ol + out_v<s>(v)), i = slot<s>(l + in_v<s>(v));
+        if (o >= SLOTS || i >= SLOTS || o != lo + so[v] || i != li + si[v]) return false;
+        if (!ONE && (o / SEC != l / LW || (s == 0 && i / SEC != l / LW))) return false;
+      }
+    }
+    return true;
+  }
+
+  const int col, lane, l0;  // this thread's column of the tile, lane, and lane of the first stage
+  T* const lds;             // the exchange region, at this thread's column
+  const T* const tw;
+  __device__ __forceinline__ TileFft(T* region, const T* tw_)
+      : col((int)(threadIdx.x % (unsigned)CW)), lane((int)(threadIdx.x / (unsigned)CW)),
+        l0(lane0((int)(threadIdx.x / (unsigned)CW))), lds(region + threadIdx.x % (unsigned)CW), tw(tw_) {}
+
+  __device__ __forceinline__ static void sync() {
+    if constexpr (ONE) wave_sync();
+    else __syncthreads();
+  }
+  template <int s, bool IN, bool PUT>
+  __device__ __forceinline__ void move(T* v) const {
+    static_assert(slots_ok<s>(), "exchange slots must split into lane base and constant, inside their sections");
+    T* p = lds + slot<s>(IN ? lane : out_l<s>(s == 0 ? l0 : lane)) * CW;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      const int k = slot<s>(IN ? in_v<s>(e) : out_v<s>(e)) * CW;
+      if constexpr (PUT) p[k] = v[e];
+      else v[e] = p[k];
+    }
+  }
+  template <int s>
+  __device__ __forceinline__ void forward_from(T* v) const {
+    B::template twiddle<s, false>(v, tw, lane);
+    B::template butterflies<s, false>(v);
+    if constexpr (s + 1 < S) {
+      if constexpr (s != 1) sync();
+      move<s, false, true>(v);
+      if constexpr (s == 0) wave_sync();
+      else sync();
+      move<s, true, false>(v);
+      wave_sync();
+      forward_from<s + 1>(v);
+    }
+  }
+  // v: values at l0 + first_c -> spectrum at lane + last_c, unnormalized
+  __device__ __forceinline__ void forward(T* v) const {
+    asm volatile("" ::: "memory");
+    forward_from<0>(v);
+  }
+  template <int s>
+  __device__ __forceinline__ void inverse_from(T* v) const {
+    B::template butterflies<s, true>(v);
+    B::template twiddle<s, true>(v, tw, lane);
+    if constexpr (s > 0) {
+      if constexpr (s > 1) sync();
+      move<s - 1, true, true>(v);
+      if constexpr (s > 1) sync();
+      else wave_sync();
+      move<s - 1, false, false>(v);
+      wave_sync();
+      inverse_from<s - 1>(v);
+    }
+  }
+  // v: spectrum at lane + last_c -> values at l0 + first_c, unnormalized
+  __device__ __forceinline__ void inverse(T* v) const {
+    asm volatile("" ::: "memory");
+    inverse_from<S - 1>(v);
   }
 };
 

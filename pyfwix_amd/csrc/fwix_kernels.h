@@ -14,40 +14,23 @@ constexpr bool size_has3(int N) { return N % 3 == 0; }
 // takes 1298 instead of 824 us per 128-plane launch.)
 constexpr int kRowWaves = 4;
 constexpr int kRowThreads = 64 * kRowWaves;
-// Column passes: 512-thread workgroups, 8 waves x CW/8 columns, with each
-// lane holding V = CW*N/512 values: 8 (2^a, N <= 512), 16 (1024) or 12 (3*2^a).
-// Two workgroups fit a CU, so one tile's loads overlap another's transforms.
 // Default register budget (waves per SIMD) of the column kernels, from timed
-// launches of every budget on MI355X: kind 0 the forward / fan-out
-// transforms, kind 1 the fan-in transforms; mode 2 the scattering terms.
-// (Every mode of a kind has the same winners so far; mode stays in the key.)
+// launches of every budget on MI355X: kind 0 the fan-out transforms, kind 1
+// the fan-in transforms; mode 2 the scattering terms.  (Every mode of a kind
+// has the same winners so far; mode stays in the key.)  The fan-out needs at most
+// 92 registers (113 at 1024 points) and is the same code at every budget but
+// for its schedule (within 3 %).  The fan-in fits 4 waves at V = 8 (16 M points,
+// 512: 223 us at 2, 215 at 4, 275 at 6 with spills); at V = 12 that budget
+// spills (192: 129 / 138 / 129 us, 384: 233 / 244 / 211 us, the third at no
+// budget, which LDS rules out; 768: 315 / 282 / 305 us); at 1024 points LDS holds
+// 3 workgroups and the budgets are equal (210 to 214 us).
 constexpr int col_wpe_default(int kind, int mode, int N) {
   const bool pow2 = !size_has3(N);
   (void)mode;
-  if (kind == 0) return (pow2 && N <= 512) ? 6 : (N == 384 || N == 768) ? 4 : 2;
+  if (kind == 0) return N == 1024 ? 2 : pow2 ? 6 : 4;
   return (pow2 && N <= 512) || N == 768 ? 4 : 2;
 }
-// 1024-point columns use 256-thread workgroups (4 waves) on 4-column tiles:
-// a 1024 x 8 tile takes 74 KB of LDS and, with the 256-VGPR budget these
-// transforms need, one 8-wave workgroup per CU, so nothing overlapped one
-// tile's loads with another's transforms; two 4-wave workgroups share a CU.
-constexpr int col_threads(int N) { return N == 1024 ? 256 : 512; }
-constexpr int col_cw(int N) {
-  if (N == 1024) return 4;
-  const int cw = (size_has3(N) ? 6144 : 4096) / N;
-  return cw < 8 ? 8 : cw;
-}
-constexpr int kColThreads = 512;
 constexpr int kThreads = 256;
-
-// LDS layouts -------------------------------------------------------------
-// Stockham exchanges write with stride R inside a batch; one pad slot every
-// 32 complex samples spreads those writes over all 64 LDS banks.
-constexpr int padded(int N) { return N + N / 32; }
-template <int N>
-struct PadLds {  // one wave's NB batches, batch-major, padded
-  __device__ __forceinline__ static int addr(int b, int i) { return b * padded(N) + i + (int)((unsigned)i >> 5); }
-};
 
 // One argument block for every step kernel (passed by value).
 struct KArgs {
@@ -67,7 +50,7 @@ struct KArgs {
   const float* tapx;       // (NX) taper weights
   const float* tapy;       // (NY)
   const float2* twx;       // (NX) stage twiddles of the row transforms (twiddle_exp)
-  const float2* twy;       // (NY) twiddles exp(-2 pi i k/NY)
+  const float2* twy;       // (NY) stage twiddles of the column transforms
   const double2* twx64;    // the same tables and taper weights in float64, for the
   const double2* twy64;    //   passes that run in float64 arithmetic (f64)
   const double* tapx64;

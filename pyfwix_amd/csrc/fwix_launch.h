@@ -41,9 +41,8 @@ struct PwArgs {
 };
 
 bool fft_size_supported(int n);
-int col_tile_width(int n);  // columns per column-pass workgroup for an n-point column FFT
 
-// fused step passes (step_kernels.hip)
+// fused step passes (row_kernels.hip, cols_fanout.hip, cols_fanin.hip, step_kernels.hip)
 hipError_t launch_rows(int kind, const KArgs& a, hipStream_t st);      // 0 fwd, 1 inv, 2 fwd+pre-taper, 3 inv+post-taper
 hipError_t launch_rows_fanout(const KArgs& a, hipStream_t st);
 hipError_t launch_rows_select(const KArgs& a, hipStream_t st);
@@ -98,8 +97,8 @@ hipError_t launch_ic_adj(float2* img, const float2* D, const float2* U, int NX, 
 // fan-out / 1 fan-in, per mode (0, 1, 2) and column length; -1 if invalid.
 int col_wpe_get(int kind, int mode, int n);
 int col_wpe_set(int kind, int mode, int n, int wpe);
-// Column layout of the n-point transforms (kind, mode as above): 0 one wave
-// per column, 1 two waves per column (n = 1024 only); -1 if invalid.
+// Column layout of the n-point transforms (kind, mode as above): 0 tiles of 8
+// columns, 1 tiles of 4 (n = 1024 only); -1 if invalid.
 int col_layout_get(int kind, int mode, int n);
 int col_layout_set(int kind, int mode, int n, int layout);
 // Layout of the K / W scratch for column length n: 1 quad-block, 0 row-major; -1 if invalid.

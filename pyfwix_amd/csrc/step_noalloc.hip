@@ -106,12 +106,12 @@ __global__ void k_step_tables(float* kx, float* ky, float* w2, float* tapx, floa
   if (i < NX) {
     kx[i] = kval(i, NX, dx);
     tapx[i] = tap(i, NX, tx);
-    twx[i] = tw(twiddle_exp(NX, false, i), NX);
+    twx[i] = tw(twiddle_exp(NX, kRow32, i), NX);
   }
   if (i < NY) {
     ky[i] = kval(i, NY, dy);
     tapy[i] = tap(i, NY, ty);
-    twy[i] = tw(i, NY);
+    twy[i] = tw(twiddle_exp(NY, kCol32, i), NY);
   }
   if (i < NW) {
     const double f = 2.0 * M_PI * (ow + (double)i * dw);
