@@ -108,6 +108,7 @@ struct ColOffs {
 // In LDS because one wait counter covers vector loads and stores: a global
 // load in the loop over the terms would wait for the term's stores or for the
 // next term's tile in flight.
+// (every thread group of a workgroup writes the same values)
 template <class F, class T>
 __device__ __forceinline__ void col_twiddles(T* twl, const T* __restrict__ tw) {
   for (int i = threadIdx.x; i < F::TW; i += F::THREADS) twl[i] = tw[i];
@@ -221,9 +222,12 @@ hipError_t dispatch_mode(int mode, Fn&& fn) {
 }
 // One column kernel per (size, mode) and, in float32, register budget (2, 4
 // or 6 waves per SIMD, col_wpe_get) and at 1024 points tile width
-// (col_layout_get); float64 arithmetic (a.f64) has one budget.
-// K<N, MODE, WPE, T, CW>::kernel
-template <template <int, int, int, class, int> class K>
+// (col_layout_get); float64 arithmetic (a.f64) has one budget.  Launches that
+// leave the chip idle split their terms (term_split): a fan-out over more
+// workgroups (each with its own forward transform), a fan-in (GROUPS) over thread groups
+// of its workgroups.  K<N, MODE, WPE, T, CW, G>::kernel
+constexpr int col_groups(int threads, int N) { return threads <= 128 || N == 256 ? 4 : 2; }
+template <template <int, int, int, class, int, int> class K, bool GROUPS>
 hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) {
   return dispatch_n(a.NY, [&](auto nc) {
     constexpr int N = decltype(nc)::value;
@@ -231,9 +235,21 @@ hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) 
       constexpr int M = decltype(mc)::value;
       auto go = [&](auto wc, auto cc, auto t) -> hipError_t {
         using T = decltype(t);
-        constexpr int CW = decltype(cc)::value;
+        constexpr int CW = decltype(cc)::value, W = decltype(wc)::value;
         using F = TileFft<N, T, CW>;
-        hipLaunchKernelGGL((K<N, M, decltype(wc)::value, T, CW>::kernel), col_grid<F>(a), dim3(F::THREADS), 0, st, a);
+        dim3 g = col_grid<F>(a), b(F::THREADS);
+        const long long waves = (long long)g.x * g.y * F::WAVES;
+        if constexpr (!GROUPS) {
+          g.z = term_split(waves, a.nterm, 4, 2048);
+        } else if constexpr (M != 2 && sizeof(T) == 8 && F::THREADS * CW < 4096) {  // (1024 x 8: two regions exceed LDS)
+          constexpr int G = col_groups(F::THREADS, N);
+          if (term_split(waves, a.nterm, G, 512) > 1) {
+            b.y = G;
+            hipLaunchKernelGGL((K<N, M, 2, T, CW, G>::kernel), g, b, 0, st, a);
+            return hipGetLastError();
+          }
+        }
+        hipLaunchKernelGGL((K<N, M, W, T, CW, 1>::kernel), g, b, 0, st, a);
         return hipGetLastError();
       };
       constexpr std::integral_constant<int, col_cw(N, true, 0)> cw64{};

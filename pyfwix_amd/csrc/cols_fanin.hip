@@ -7,14 +7,19 @@
 
 namespace fwix {
 
-// (T: arithmetic type of the transforms, float2 or double2)
-template <int N, int MODE, int WPE, class T, int CWX>
-__global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgpu_waves_per_eu(WPE))) void k_cols_fanin(KArgs a) {
+// (T: arithmetic type of the transforms, float2 or double2; G: groups of
+// threads that share a tile's terms, group g taking every G-th, their sums
+// added in group order)
+template <int N, int MODE, int WPE, class T, int CWX, int G>
+__global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS * G)) __attribute__((amdgpu_waves_per_eu(WPE))) void k_cols_fanin(KArgs a) {
   using F = TileFft<N, T, CWX>;
   using S = real_of<T>;
-  __shared__ __align__(16) T region[F::SMEM];
+  constexpr int SM = G > 1 && F::SMEM < N * F::CW ? N * F::CW : F::SMEM;
+  __shared__ __align__(16) T regions[G * SM];
   __shared__ __align__(16) T twl[F::TW];
   __shared__ uint32_t rmk[N];
+  const int g = G > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.y) : 0;
+  T* region = regions + g * SM;
   const F f(region, twl);
   int p, c0;
   col_tile<F>(p, c0);
@@ -32,7 +37,8 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
   S k2v[F::V];
   column_k2(k2v, f, a, c0);
   const S w2 = a.w2[iw];
-  F::sync();
+  if constexpr (G > 1) __syncthreads();
+  else F::sync();
   // the next term's tile is fetched into registers during this term's
   // transform, as it is stored (float32)
   float2 nxt[F::V];
@@ -50,39 +56,64 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
   T acc[F::V];
 #pragma unroll
   for (int e = 0; e < F::V; ++e) acc[e] = cz<T>();
-  int r = masked ? next_bit(live, -1) : 0;
+  // the k-th term after r, rend or more when there is none
+  auto after = [&](int r, int k) {
+    for (int i = 0; i < k && r < rend; ++i) r = masked ? next_bit(live, r) : r + 1;
+    return r;
+  };
+  int lead = masked ? next_bit(live, -1) : 0;  // group 0's term: the groups wait for each other, so all go as far
+  int r = after(lead, g);
   if (r < rend) fetch(r);
-  while (r < rend) {
+  while (lead < rend) {
+    lead = after(lead, G);
+    if (G > 1 && F::ONE && r >= rend) break;  // no waits in a tile of one wave
     T x[F::V];
 #pragma unroll
-    for (int e = 0; e < F::V; ++e) x[e] = from_f2<T>(nxt[e]);
-    const int rn = masked ? next_bit(live, r) : r + 1;
+    for (int e = 0; e < F::V; ++e) x[e] = G > 1 && r >= rend ? cz<T>() : from_f2<T>(nxt[e]);
+    const int rn = after(r, G);
     if (rn < rend) fetch(rn);
     f.forward(x);
-    const TermMult<MODE, T> tm(a, r, iw, w2);
-    auto mult = [&](auto real) {
+    if (G == 1 || r < rend) {
+      const TermMult<MODE, T> tm(a, r, iw, w2);
+      auto mult = [&](auto real) {
 #pragma unroll
-      for (int e = 0; e < F::V; ++e) acc[e] = cadd(acc[e], tm.template apply<decltype(real)::value>(x[e], k2v[e]));
-    };
-    if (tm.real) mult(std::true_type{});
-    else mult(std::false_type{});
+        for (int e = 0; e < F::V; ++e) acc[e] = cadd(acc[e], tm.template apply<decltype(real)::value>(x[e], k2v[e]));
+      };
+      if (tm.real) mult(std::true_type{});
+      else mult(std::false_type{});
+    }
     r = rn;
+  }
+  if constexpr (G > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < F::V; ++e)
+      if (g > 0) region[e * F::THREADS + threadIdx.x] = acc[e];
+    __syncthreads();
+    if (F::ONE && g > 0) return;
+    // the other groups run along to the end for its waits
+#pragma unroll
+    for (int h = 1; h < G; ++h)
+#pragma unroll
+      for (int e = 0; e < F::V; ++e)
+        if (g == 0) acc[e] = cadd(acc[e], regions[h * SM + e * F::THREADS + threadIdx.x]);
   }
   const S s2 = a.scale;
 #pragma unroll
   for (int e = 0; e < F::V; ++e) acc[e] = cscale(acc[e], s2);
   f.inverse(acc);
+  if (g > 0) return;
   const PlaneBuf K(a.K + pb, plane_bytes(a));
 #pragma unroll
   for (int e = 0; e < F::V; ++e) K.store(to_f2(acc[e]), o.voff(e), o.soff(e));
 }
 
-template <int N, int MODE, int WPE, class T, int CWX>
+template <int N, int MODE, int WPE, class T, int CWX, int G>
 struct FanIn {
-  static constexpr auto kernel = &k_cols_fanin<N, MODE, WPE, T, CWX>;
+  static constexpr auto kernel = &k_cols_fanin<N, MODE, WPE, T, CWX, G>;
 };
 hipError_t launch_cols_fanin(int mode, const KArgs& a, hipStream_t st) {
-  return launch_col_terms<FanIn>(1, mode, a, st);
+  return launch_col_terms<FanIn, true>(1, mode, a, st);
 }
 
 }  // namespace fwix

@@ -19,6 +19,10 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
   int p, c0;
   col_tile<F>(p, c0);
   const size_t pb = (size_t)p * a.NX * N;
+  const int iw = plane_iw(a, p);
+  const int im = model_iw_any(a, iw);
+  const uint32_t* rm = (MODE != 2 && a.rowmask) ? a.rowmask + im * a.NY : nullptr;
+  const uint32_t pm = (MODE != 2 && a.planemask) ? a.planemask[im] : 0xffffffffu;
   const ColOffs<F, true> o(f, c0, a.NX, a.quad != 0);
   T spec[F::V];
   {
@@ -26,10 +30,6 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
 #pragma unroll
     for (int e = 0; e < F::V; ++e) spec[e] = from_f2<T>(K.load(o.voff(e), o.soff(e)));
   }
-  const int iw = plane_iw(a, p);
-  const int im = model_iw_any(a, iw);
-  const uint32_t* rm = (MODE != 2 && a.rowmask) ? a.rowmask + im * a.NY : nullptr;
-  const uint32_t pm = (MODE != 2 && a.planemask) ? a.planemask[im] : 0xffffffffu;
   col_twiddles<F>(twl, twy_of(a, (T*)nullptr));
   col_row_masks<F, N>(rmk, rm);
   S k2v[F::V];
@@ -40,8 +40,12 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
   const S s2 = a.scale;  // 1/NY: forward and inverse column normalisation together
 #pragma unroll
   for (int e = 0; e < F::V; ++e) spec[e] = cscale(spec[e], s2);
+  // part blockIdx.z takes every gridDim.z-th of the plane's terms
+  int turn = (int)blockIdx.z;
   for (int r = 0; r < a.nterm; ++r) {
     if (r < 32 && !((pm >> r) & 1u)) continue;  // reference absent from the plane: W_r is never read
+    if (turn-- != 0) continue;
+    turn = (int)gridDim.z - 1;
     const TermMult<MODE, T> tm(a, r, iw, w2);
     T x[F::V];
     auto mult = [&](auto real) {
@@ -64,12 +68,12 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
   }
 }
 
-template <int N, int MODE, int WPE, class T, int CWX>
+template <int N, int MODE, int WPE, class T, int CWX, int G>
 struct FanOut {
   static constexpr auto kernel = &k_cols_fanout<N, MODE, WPE, T, CWX>;
 };
 hipError_t launch_cols_fanout(int mode, const KArgs& a, hipStream_t st) {
-  return launch_col_terms<FanOut>(0, mode, a, st);
+  return launch_col_terms<FanOut, false>(0, mode, a, st);
 }
 
 }  // namespace fwix

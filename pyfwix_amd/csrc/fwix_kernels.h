@@ -127,12 +127,13 @@ struct RowLane {
   int l, b, rb, nrows;
   bool live;
   int iw, iy;  // frequency plane and row of the plane (of the last row for dead lanes)
-  __device__ __forceinline__ explicit RowLane(const KArgs& a) {
+  // groups: this many consecutive waves share the rows of one
+  __device__ __forceinline__ explicit RowLane(const KArgs& a, int groups = 1) {
     const int lane = (int)threadIdx.x & 63;
     l = (int)((unsigned)lane % F::L);
     b = (int)((unsigned)lane / F::L);
     nrows = a.np * a.NY;
-    rb = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * kRowWaves + (threadIdx.x >> 6)) * F::NB));
+    rb = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * kRowWaves + (threadIdx.x >> 6)) / groups * F::NB));
     const int lr = rb + b;
     live = lr < nrows;
     const int row = live ? lr : nrows - 1;

@@ -20,10 +20,33 @@ hipError_t dispatch_n(int n, Fn&& fn) {
   }
 }
 
+// (groups: waves that share the rows of one wave, see k_rows_select)
 template <int N, class T>
-inline dim3 row_grid(int nrows) {
-  constexpr int per = kRowWaves * LaneFft<N, T>::NB;
+inline dim3 row_grid(int nrows, int groups = 1) {
+  const int per = kRowWaves / groups * LaneFft<N, T>::NB;
   return dim3((nrows + per - 1) / per);
+}
+template <int N, class T>
+inline long long row_waves(int nrows) {
+  return (nrows + LaneFft<N, T>::NB - 1) / LaneFft<N, T>::NB;
+}
+// Into how many parts (at most `most`) a launch of `waves` waves splits the
+// terms each of its waves would work through.  A launch with few waves takes
+// as long as one wave's chain of transforms: at 96 x 128 x 24 planes (384
+// column and 576 row waves on 1024 SIMDs, 4 terms) the chip is 10 % busy and
+// splitting takes the fan-out columns from 14.9 to 10.9 us, the fan-in from
+// 13.6 to 10.5, the fan-out rows from 10.9 to 8.6, the select from 8.2 to 7.2.
+// Fan-outs repeat the shared transform in every part and pay below two waves
+// per SIMD (`limit` 2048; 192 x 192 x 32 planes, 1536 waves: 18.4 -> 16.1 us;
+// 256 x 256 x 32, 4096 waves, split in 2: the Born pass 13 % slower).  Where the
+// parts meet in LDS it takes less than one: 1024 for the select (192 x 192 x 16,
+// 768 waves: 11.5 -> 10.5 us), 512 for the fan-in, whose groups also wait for each
+// other (192 x 192 x 4, 192 waves: 14.3 -> 12.4 us; x 16, 768 waves: 17.4 -> 22.6).
+inline int term_split(long long waves, int nterm, int most, int limit) {
+  if (waves >= limit || nterm < 2) return 1;
+  const long long z = (2048 + waves - 1) / waves;
+  const int m = nterm < most ? nterm : most;
+  return z < m ? (int)z : m;
 }
 // Argument block of the point-wise operator kernels.
 struct PwArgs {

@@ -135,8 +135,11 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_fanout(KArgs a) {
   if (w.empty()) return;
   const real_of<T> s = a.scale;
   const uint32_t wm = wave_row_mask<N, T, MAP>(a, w);
+  int turn = (int)blockIdx.y;  // part blockIdx.y takes every gridDim.y-th of the wave's references
   for (int r = 0; r < a.nref; ++r) {
     if (r < 32 && !((wm >> r) & 1u)) continue;  // rows without reference r: the column pass reads zeros
+    if (turn-- != 0) continue;
+    turn = (int)gridDim.y - 1;
     T x[F::V];
 #pragma unroll
     for (int e = 0; e < F::V; ++e) x[e] = (lab.at(e) == r) ? u[e] : cz<T>();
@@ -151,12 +154,16 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_fanout(KArgs a) {
 // KNEXT: also K = scale * F_x(taper * out) (quad-block), the first row pass of
 // a next step that propagates out further: one transform more here instead of
 // a pass that reads out back.
-template <int N, bool MAP, bool KNEXT = false>
+// G: waves that share the rows of one, each taking every G-th of their
+// references (launches that leave the chip idle, term_split).
+template <int N, bool MAP, bool KNEXT = false, int G = 1>
 __global__ __launch_bounds__(kRowThreads) void k_rows_select(KArgs a) {
   using F = LaneFft<N>;
   __shared__ float2 lds[kRowWaves * F::NB * F::STRIDE];
   __shared__ float2 twl[F::TW];
-  const RowLane<N, float2> w(a);
+  static_assert(kRowWaves % G == 0, "a workgroup holds whole groups");
+  const RowLane<N, float2> w(a, G);
+  const int g = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) % G);
   float2* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   Labels<F::V> lab;
   float2 acc[F::V];
@@ -178,17 +185,21 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_select(KArgs a) {
   // this one's transform, except at 16 values per lane or more, where holding
   // it would cost a wave of occupancy
   constexpr bool PREFETCH = F::V < 16;
-  int r = a.rowmask ? next_bit(live, -1) : 0;
   const int rend = a.rowmask ? 32 : a.nref;
+  auto after = [&](int r, int k) {  // the k-th reference after r, rend or more when there is none
+    for (int i = 0; i < k && r < rend; ++i) r = a.rowmask ? next_bit(live, r) : r + 1;
+    return r;
+  };
+  int r = after(a.rowmask ? next_bit(live, -1) : 0, g);
   if (r < rend) fetch(r);
   row_twiddles<N>(twl, a.twx);
   __syncthreads();
-  if (w.empty()) return;
+  if (G == 1 && w.empty()) return;
   while (r < rend) {
     float2 x[F::V];
 #pragma unroll
     for (int e = 0; e < F::V; ++e) x[e] = nxt[e];
-    const int rn = a.rowmask ? next_bit(live, r) : r + 1;
+    const int rn = after(r, G);
     if (PREFETCH && rn < rend) fetch(rn);
     F::template run<true>(x, line, twl, w.l);
     if (!PREFETCH && rn < rend) fetch(rn);
@@ -197,6 +208,19 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_select(KArgs a) {
     for (int e = 0; e < F::V; ++e)
       if (lab.at(e) == r) acc[e] = x[e];
     r = rn;
+  }
+  if constexpr (G > 1) {  // the first wave of a group gathers the nodes of the others (each node has one owner)
+    wave_sync();
+#pragma unroll
+    for (int e = 0; e < F::V; ++e)
+      if (g > 0) line[w.l + F::first_c(e)] = acc[e];
+    __syncthreads();
+    if (g > 0 || w.empty()) return;
+#pragma unroll
+    for (int h = 1; h < G; ++h)
+#pragma unroll
+      for (int e = 0; e < F::V; ++e) acc[e] = cadd(acc[e], line[h * F::NB * F::STRIDE + w.l + F::first_c(e)]);
+    wave_sync();
   }
   const float s = a.scale;
   const RowBuf<N, float2> out(a.out, w, false);
@@ -294,30 +318,32 @@ hipError_t launch_rows(int kind, const KArgs& a, hipStream_t st) {
 hipError_t launch_rows_fanout(const KArgs& a, hipStream_t st) {
   return dispatch_n(a.NX, [&](auto nc) -> hipError_t {
     constexpr int N = decltype(nc)::value;
-    const dim3 g = row_grid<N, float2>(a.np * a.NY), g64 = row_grid<N, double2>(a.np * a.NY);
-    if (a.f64) {
-      if (a.mplane) hipLaunchKernelGGL((k_rows_fanout<N, true, double2>), g64, dim3(kRowThreads), 0, st, a);
-      else hipLaunchKernelGGL((k_rows_fanout<N, false, double2>), g64, dim3(kRowThreads), 0, st, a);
-    } else {
-      if (a.mplane) hipLaunchKernelGGL((k_rows_fanout<N, true>), g, dim3(kRowThreads), 0, st, a);
-      else hipLaunchKernelGGL((k_rows_fanout<N, false>), g, dim3(kRowThreads), 0, st, a);
-    }
-    return hipGetLastError();
+    auto go = [&](auto map, auto t) {
+      using T = decltype(t);
+      dim3 g = row_grid<N, T>(a.np * a.NY);
+      g.y = term_split(row_waves<N, T>(a.np * a.NY), a.nref, 4, 2048);
+      hipLaunchKernelGGL((k_rows_fanout<N, decltype(map)::value, T>), g, dim3(kRowThreads), 0, st, a);
+      return hipGetLastError();
+    };
+    if (a.f64) return a.mplane ? go(std::true_type{}, double2{}) : go(std::false_type{}, double2{});
+    return a.mplane ? go(std::true_type{}, float2{}) : go(std::false_type{}, float2{});
   });
 }
 
 hipError_t launch_rows_select(const KArgs& a, hipStream_t st) {
   return dispatch_n(a.NX, [&](auto nc) -> hipError_t {
     constexpr int N = decltype(nc)::value;
-    const dim3 g = row_grid<N, float2>(a.np * a.NY);
-    if (a.knext) {
-      if (a.mplane) hipLaunchKernelGGL((k_rows_select<N, true, true>), g, dim3(kRowThreads), 0, st, a);
-      else hipLaunchKernelGGL((k_rows_select<N, false, true>), g, dim3(kRowThreads), 0, st, a);
-    } else {
-      if (a.mplane) hipLaunchKernelGGL((k_rows_select<N, true>), g, dim3(kRowThreads), 0, st, a);
-      else hipLaunchKernelGGL((k_rows_select<N, false>), g, dim3(kRowThreads), 0, st, a);
-    }
-    return hipGetLastError();
+    auto go = [&](auto map, auto knext) {
+      constexpr bool M = decltype(map)::value, K = decltype(knext)::value;
+      const int nrows = a.np * a.NY;
+      const bool split = term_split(row_waves<N, float2>(nrows), a.nref, kRowWaves, 1024) > 1;
+      const dim3 g = row_grid<N, float2>(nrows, split ? kRowWaves : 1);
+      if (split) hipLaunchKernelGGL((k_rows_select<N, M, K, kRowWaves>), g, dim3(kRowThreads), 0, st, a);
+      else hipLaunchKernelGGL((k_rows_select<N, M, K>), g, dim3(kRowThreads), 0, st, a);
+      return hipGetLastError();
+    };
+    if (a.knext) return a.mplane ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
+    return a.mplane ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
   });
 }
 

@@ -73,3 +73,33 @@ def test_float64_columns_of_every_kind(dev, ny):
     from test_gpu_born import _born_vs_oracle
     errs, _ = _born_vs_oracle(dev, (48, ny, 2, 40, ny - 8), 6.0, precision=FWIX_PREC_F64_SCATTER)
     assert max(errs) < TOL_WFLD, errs
+
+
+@pytest.mark.parametrize("nx,ny", [(16, 12), (96, 64), (128, 192), (256, 256), (384, 384), (512, 768), (48, 1024)])
+@pytest.mark.parametrize("masks", [True, False])
+def test_small_launches_split_their_terms(dev, nx, ny, masks):
+    """A plane on its own (few waves: its references shared out over
+    workgroups, thread groups or waves) and among so many that nothing is split: the
+    same step up to the order in which the references' spectra are added
+    (2^-24 per addition; 1e-6 relative).  nref = 40 runs without presence masks."""
+    import torch
+    from pyfwix_amd.ops import FWIX_NSPS, FWIX_PSPI, OneStep
+    rng = np.random.default_rng(nx + ny)
+    nref = 5 if masks else 40
+    many = max(2, min(400, (6 << 20) // (nx * ny)))
+    sref = (1.0 / rng.uniform(1500, 3000, (1, nref, 1)) ** 2).astype(np.complex64)
+    lab = rng.integers(0, nref, (1, 1, ny, nx)).astype(np.uint8)
+    lab[0, 0, : ny // 2] = nref - 1
+    x = crand(rng, (1, 1, ny, nx))
+    for method in (FWIX_PSPI, FWIX_NSPS):
+        out = []
+        for nw in (1, many):
+            op = OneStep(method, dims_of(grid(nx, ny, nw, 1, nz=1, dw=0.0)), nref=nref, taperx=2, tapery=3)
+            op.set_refs(_t(np.repeat(sref, nw, 2), dev), _t(np.repeat(lab, nw, 1), dev, np.uint8))
+            op.set_depth(0)
+            u = _t(np.repeat(x, nw, 1), dev)
+            f, a = torch.zeros_like(u), torch.zeros_like(u)
+            op.forward(False, u, f)
+            op.adjoint(False, a, u)
+            out.append((f[0, -1].cpu().numpy(), a[0, -1].cpu().numpy()))
+        assert rel(out[0][0], out[1][0]) < 1e-6 and rel(out[0][1], out[1][1]) < 1e-6, method
