@@ -16,7 +16,8 @@
 // per element.  Before -> now, us per launch: fan-out 512^2 x 64 planes 175 ->
 // 143, 384^2 x 200 375 -> 270, 1024^2 x 128 1012 -> 884, 192 x 384 x 26 (complex
 // slowness) 92 -> 50, 96 x 128 x 24 25 -> 15; fan-in 212 -> 180, 572 -> 335, 1237 -> 1044,
-// 121 -> 53, 25 -> 14; float64 768^2 x 6 fan-out 222 -> 134, fan-in 443 -> 272.
+// 121 -> 53, 25 -> 14; float64 768^2 x 6 fan-out 222 -> 95, fan-in 443 -> 102 (with sincospi and k^2 not held: 134 and
+// 272 before, 117 registers spilled).
 #pragma once
 #include "fwix_kernels.h"
 #include "fwix_launch.h"
@@ -162,8 +163,15 @@ struct TermMult {
       for (int i = 0; i < r; ++i) m *= q;
       return cscale(x, m);
     } else if constexpr (sizeof(S) == 8) {
-      if constexpr (!REAL) return cmul(x, ps_general64<MULT>(wsre - k2, b, dz));
-      else return cmul(x, ps_real64<MULT>(wsre - k2, dz));
+      if constexpr (!REAL) {
+        return cmul(x, ps_general64<MULT>(wsre - k2, b, dz));
+      } else {
+        const S a = wsre - k2, q = sqrt(fabs(a));
+        if (a < 0) return cscale(x, exp(-q * dz));
+        S sn, cs;
+        sincospi(q * (dz * kInvPi), &sn, &cs);
+        return cmul(x, CX<T>::mk(cs, MULT == 0 ? -sn : sn));
+      }
     } else if constexpr (!REAL) {
       return cmul(x, ps_general<MULT>(wsre - k2, b, dz));
     } else {
@@ -181,20 +189,37 @@ struct TermMult {
     }
   }
 };
-// k^2 = kx^2 + ky^2 at this thread's samples after a forward transform
-// (the positions of the last stage); loop-invariant over the terms.
-template <class F, class S>
-__device__ __forceinline__ void column_k2(S* k2v, const F& f, const KArgs& a, int c0) {
-  const int col = c0 + f.col;
-  const S kxv = a.kx[col < a.NX ? col : 0];
-  const float* ky = a.ky + f.lane;
+// k^2 = kx^2 + ky^2 at this thread's samples after a forward transform (the
+// positions of the last stage).  In float32 held in registers over the terms;
+// in float64, where that would be 2 V registers of kernels at their budget,
+// formed from the wavenumbers staged in LDS (the caller synchronises).
+template <class F, int N, class S>
+struct ColumnK2 {
+  static constexpr bool HELD = sizeof(S) == 4;
+  S v[HELD ? F::V : 1];
+  const float* ky;
+  __device__ __forceinline__ ColumnK2(const F& f, const KArgs& a, int c0, float* lds) {
+    const int col = c0 + f.col;
+    const S kxv = a.kx[col < a.NX ? col : 0];
+    if constexpr (HELD) {
+      ky = a.ky + f.lane;
 #pragma unroll
-  for (int e = 0; e < F::V; ++e) {
-    const S kyv = ky[F::last_c(e)];
-    if constexpr (sizeof(S) == 8) k2v[e] = fma(kxv, kxv, kyv * kyv);
-    else k2v[e] = fmaf(kxv, kxv, kyv * kyv);
+      for (int e = 0; e < F::V; ++e) {
+        const S kyv = ky[F::last_c(e)];
+        v[e] = fmaf(kxv, kxv, kyv * kyv);
+      }
+    } else {
+      for (int i = threadIdx.x; i < N; i += F::THREADS) lds[i] = a.ky[i];
+      ky = lds + f.lane;
+      v[0] = kxv;
+    }
   }
-}
+  __device__ __forceinline__ S at(int e) const {
+    if constexpr (HELD) return v[e];
+    const S kyv = ky[F::last_c(e)];
+    return fma(v[0], v[0], kyv * kyv);
+  }
+};
 
 // ------------------------------------------------------------------ launch geometry
 template <class F>

@@ -34,8 +34,8 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS * G)) __attribute__((a
   const int rend = masked ? 32 : a.nterm;
   col_twiddles<F>(twl, twy_of(a, (T*)nullptr));
   col_row_masks<F, N>(rmk, rm);
-  S k2v[F::V];
-  column_k2(k2v, f, a, c0);
+  __shared__ float kyl[sizeof(S) == 8 ? N : 1];
+  const ColumnK2<F, N, S> k2(f, a, c0, kyl);
   const S w2 = a.w2[iw];
   if constexpr (G > 1) __syncthreads();
   else F::sync();
@@ -77,7 +77,7 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS * G)) __attribute__((a
       const TermMult<MODE, T> tm(a, r, iw, w2);
       auto mult = [&](auto real) {
 #pragma unroll
-        for (int e = 0; e < F::V; ++e) acc[e] = cadd(acc[e], tm.template apply<decltype(real)::value>(x[e], k2v[e]));
+        for (int e = 0; e < F::V; ++e) acc[e] = cadd(acc[e], tm.template apply<decltype(real)::value>(x[e], k2.at(e)));
       };
       if (tm.real) mult(std::true_type{});
       else mult(std::false_type{});

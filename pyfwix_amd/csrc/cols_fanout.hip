@@ -32,8 +32,8 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
   }
   col_twiddles<F>(twl, twy_of(a, (T*)nullptr));
   col_row_masks<F, N>(rmk, rm);
-  S k2v[F::V];
-  column_k2(k2v, f, a, c0);
+  __shared__ float kyl[sizeof(S) == 8 ? N : 1];
+  const ColumnK2<F, N, S> k2(f, a, c0, kyl);
   F::sync();
   f.forward(spec);
   const S w2 = a.w2[iw];
@@ -50,7 +50,7 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
     T x[F::V];
     auto mult = [&](auto real) {
 #pragma unroll
-      for (int e = 0; e < F::V; ++e) x[e] = tm.template apply<decltype(real)::value>(spec[e], k2v[e]);
+      for (int e = 0; e < F::V; ++e) x[e] = tm.template apply<decltype(real)::value>(spec[e], k2.at(e));
     };
     if (tm.real) mult(std::true_type{});
     else mult(std::false_type{});
