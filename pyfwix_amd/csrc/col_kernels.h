@@ -105,7 +105,8 @@ struct ColOffs {
 };
 
 // this workgroup's copy of the column transforms' twiddle table and of the
-// plane's row masks (all set when masks are off); the caller synchronises.
+// plane's row masks, inverted (absent references set; none when masks are off);
+// the caller synchronises.
 // In LDS because one wait counter covers vector loads and stores: a global
 // load in the loop over the terms would wait for the term's stores or for the
 // next term's tile in flight.
@@ -116,7 +117,11 @@ __device__ __forceinline__ void col_twiddles(T* twl, const T* __restrict__ tw) {
 }
 template <class F, int N>
 __device__ __forceinline__ void col_row_masks(uint32_t* rml, const uint32_t* __restrict__ rm) {
-  for (int i = threadIdx.x; i < N; i += F::THREADS) rml[i] = rm ? rm[i] : 0xffffffffu;
+  for (int i = threadIdx.x; i < N; i += F::THREADS) rml[i] = rm ? ~rm[i] : 0u;
+}
+// offset off of an element whose row has reference r (< 32), else kOff
+__device__ __forceinline__ unsigned off_if(uint32_t absent, int r, unsigned off) {
+  return off | ((absent << (31 - r)) & kOff);
 }
 // Reference slowness r of the plane, by a scalar load (through a
 // constant-address-space pointer): that load waits on the scalar counter
@@ -154,26 +159,38 @@ struct TermMult {
       iw2 = 0;
     }
   }
-  // x times the multiplier at k2
-  template <bool REAL>
-  __device__ __forceinline__ T apply(T x, S k2) const {
+  // x times the multiplier at k2, plus acc where ADD
+  template <bool ADD>
+  __device__ __forceinline__ static T times(T x, S m, T acc) {
+    if constexpr (!ADD) return cscale(x, m);
+    else return CX<T>::mk(fma_(x.x, m, acc.x), fma_(x.y, m, acc.y));
+  }
+  template <bool ADD>
+  __device__ __forceinline__ static T times(T x, T m, T acc) {
+    if constexpr (!ADD) return cmul(x, m);
+    else return CX<T>::mk(fma_(x.x, m.x, fma_(-x.y, m.y, acc.x)), fma_(x.x, m.y, fma_(x.y, m.x, acc.y)));
+  }
+  __device__ __forceinline__ static float fma_(float a, float b, float c) { return fmaf(a, b, c); }
+  __device__ __forceinline__ static double fma_(double a, double b, double c) { return fma(a, b, c); }
+  template <bool REAL, bool ADD>
+  __device__ __forceinline__ T apply(T x, S k2, T acc) const {
     if constexpr (MULT == 2) {
       const S q = sizeof(S) == 8 ? k2 / w2 : k2 * iw2;
       S m = q;
       for (int i = 0; i < r; ++i) m *= q;
-      return cscale(x, m);
+      return times<ADD>(x, m, acc);
     } else if constexpr (sizeof(S) == 8) {
       if constexpr (!REAL) {
-        return cmul(x, ps_general64<MULT>(wsre - k2, b, dz));
+        return times<ADD>(x, ps_general64<MULT>(wsre - k2, b, dz), acc);
       } else {
         const S a = wsre - k2, q = sqrt(fabs(a));
-        if (a < 0) return cscale(x, exp(-q * dz));
+        if (a < 0) return times<ADD>(x, exp(-q * dz), acc);
         S sn, cs;
         sincospi(q * (dz * kInvPi), &sn, &cs);
-        return cmul(x, CX<T>::mk(cs, MULT == 0 ? -sn : sn));
+        return times<ADD>(x, CX<T>::mk(cs, MULT == 0 ? -sn : sn), acc);
       }
     } else if constexpr (!REAL) {
-      return cmul(x, ps_general<MULT>(wsre - k2, b, dz));
+      return times<ADD>(x, ps_general<MULT>(wsre - k2, b, dz), acc);
     } else {
       // Past the evanescent boundary the multiplier is real and needs no sine
       // or cosine.  A wave's samples are neighbours in (kx, ky), so most
@@ -181,21 +198,23 @@ struct TermMult {
       // 3-15 % of the plane): one test of the wave skips both.
       const float a = wsre - k2, t = __builtin_amdgcn_sqrtf(fabsf(a)) * dz;
       const float e = __expf(-t);
-      if (__builtin_amdgcn_ballot_w64(a >= 0.f) == 0) return cscale(x, e);
+      if (__builtin_amdgcn_ballot_w64(a >= 0.f) == 0) return times<ADD>(x, e, acc);
       float sn, cs;
       fast_sincos(t, &sn, &cs);
       const float2 m = a >= 0.f ? make_float2(cs, MULT == 0 ? -sn : sn) : make_float2(e, 0.f);
-      return cmul(x, m);
+      return times<ADD>(x, m, acc);
     }
   }
 };
 // k^2 = kx^2 + ky^2 at this thread's samples after a forward transform (the
-// positions of the last stage).  In float32 held in registers over the terms;
-// in float64, where that would be 2 V registers of kernels at their budget,
-// formed from the wavenumbers staged in LDS (the caller synchronises).
-template <class F, int N, class S>
+// positions of the last stage): HELD in registers over the terms, or formed
+// from the wavenumbers staged in LDS (the caller synchronises) where those registers
+// cost waves.  Float64 kernels are at their budget; the float32 fan-in with V = 12 goes
+// from 145 to 126 registers at 384 points, a fourth wave per SIMD, and from 128 with
+// 15 spilled to 126 at 768 (8 references, 34 planes: 543 -> 466 us); with V = 8 the wave
+// more is not reached (512: 215 us held, 222 not).
+template <class F, int N, class S, bool HELD>
 struct ColumnK2 {
-  static constexpr bool HELD = sizeof(S) == 4;
   S v[HELD ? F::V : 1];
   const float* ky;
   __device__ __forceinline__ ColumnK2(const F& f, const KArgs& a, int c0, float* lds) {
@@ -206,7 +225,8 @@ struct ColumnK2 {
 #pragma unroll
       for (int e = 0; e < F::V; ++e) {
         const S kyv = ky[F::last_c(e)];
-        v[e] = fmaf(kxv, kxv, kyv * kyv);
+        if constexpr (sizeof(S) == 8) v[e] = fma(kxv, kxv, kyv * kyv);
+        else v[e] = fmaf(kxv, kxv, kyv * kyv);
       }
     } else {
       for (int i = threadIdx.x; i < N; i += F::THREADS) lds[i] = a.ky[i];
@@ -217,7 +237,8 @@ struct ColumnK2 {
   __device__ __forceinline__ S at(int e) const {
     if constexpr (HELD) return v[e];
     const S kyv = ky[F::last_c(e)];
-    return fma(v[0], v[0], kyv * kyv);
+    if constexpr (sizeof(S) == 8) return fma(v[0], v[0], kyv * kyv);
+    else return fmaf(v[0], v[0], kyv * kyv);
   }
 };
 

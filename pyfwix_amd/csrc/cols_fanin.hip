@@ -7,11 +7,22 @@
 
 namespace fwix {
 
+// Waves per SIMD the kernel is compiled for under a budget.  LDS admits 3 at
+// 1024 points: 3 (168 registers, 10 spilled) beats 2 for the phase-shift terms (1024^2 x 16
+// planes, 202 against 214 us), not for the Taylor terms (75 against 73).  At 384
+// points it admits 4, which the scheduler then has to aim at (219 against 227 us, Taylor terms 70
+// against 78).
+constexpr int fanin_waves(int n, int mode, int wpe, bool f64) {
+  if (f64) return 2;
+  if (n == 1024) return mode == 2 ? 2 : 3;
+  return n == 384 && wpe < 4 ? 4 : wpe;
+}
+
 // (T: arithmetic type of the transforms, float2 or double2; G: groups of
 // threads that share a tile's terms, group g taking every G-th, their sums
 // added in group order)
 template <int N, int MODE, int WPE, class T, int CWX, int G>
-__global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS * G)) __attribute__((amdgpu_waves_per_eu(WPE))) void k_cols_fanin(KArgs a) {
+__global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS * G)) __attribute__((amdgpu_waves_per_eu(fanin_waves(N, MODE, WPE, sizeof(T) == 16)))) void k_cols_fanin(KArgs a) {
   using F = TileFft<N, T, CWX>;
   using S = real_of<T>;
   constexpr int SM = G > 1 && F::SMEM < N * F::CW ? N * F::CW : F::SMEM;
@@ -34,8 +45,9 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS * G)) __attribute__((a
   const int rend = masked ? 32 : a.nterm;
   col_twiddles<F>(twl, twy_of(a, (T*)nullptr));
   col_row_masks<F, N>(rmk, rm);
-  __shared__ float kyl[sizeof(S) == 8 ? N : 1];
-  const ColumnK2<F, N, S> k2(f, a, c0, kyl);
+  constexpr bool HELD = sizeof(S) == 4 && F::V != 12;
+  __shared__ float kyl[HELD ? 1 : N];
+  const ColumnK2<F, N, S, HELD> k2(f, a, c0, kyl);
   const S w2 = a.w2[iw];
   if constexpr (G > 1) __syncthreads();
   else F::sync();
@@ -47,7 +59,7 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS * G)) __attribute__((a
     if (masked) {
 #pragma unroll
       for (int e = 0; e < F::V; ++e)
-        nxt[e] = W.load((rmk[f.l0 + F::first_c(e)] >> r) & 1u ? o.voff(e) : kOff, o.soff(e));
+        nxt[e] = W.load(off_if(rmk[f.l0 + F::first_c(e)], r, o.voff(e)), o.soff(e));
     } else {
 #pragma unroll
       for (int e = 0; e < F::V; ++e) nxt[e] = W.load(o.voff(e), o.soff(e));
@@ -77,7 +89,7 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS * G)) __attribute__((a
       const TermMult<MODE, T> tm(a, r, iw, w2);
       auto mult = [&](auto real) {
 #pragma unroll
-        for (int e = 0; e < F::V; ++e) acc[e] = cadd(acc[e], tm.template apply<decltype(real)::value>(x[e], k2.at(e)));
+        for (int e = 0; e < F::V; ++e) acc[e] = tm.template apply<decltype(real)::value, true>(x[e], k2.at(e), acc[e]);
       };
       if (tm.real) mult(std::true_type{});
       else mult(std::false_type{});

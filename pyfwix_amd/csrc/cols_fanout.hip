@@ -32,8 +32,9 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
   }
   col_twiddles<F>(twl, twy_of(a, (T*)nullptr));
   col_row_masks<F, N>(rmk, rm);
-  __shared__ float kyl[sizeof(S) == 8 ? N : 1];
-  const ColumnK2<F, N, S> k2(f, a, c0, kyl);
+  constexpr bool HELD = sizeof(S) == 4;
+  __shared__ float kyl[HELD ? 1 : N];
+  const ColumnK2<F, N, S, HELD> k2(f, a, c0, kyl);
   F::sync();
   f.forward(spec);
   const S w2 = a.w2[iw];
@@ -50,7 +51,7 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
     T x[F::V];
     auto mult = [&](auto real) {
 #pragma unroll
-      for (int e = 0; e < F::V; ++e) x[e] = tm.template apply<decltype(real)::value>(spec[e], k2.at(e));
+      for (int e = 0; e < F::V; ++e) x[e] = tm.template apply<decltype(real)::value, false>(spec[e], k2.at(e), spec[e]);
     };
     if (tm.real) mult(std::true_type{});
     else mult(std::false_type{});
@@ -60,7 +61,7 @@ __global__ __launch_bounds__((TileFft<N, T, CWX>::THREADS)) __attribute__((amdgp
       // only the rows where the reference is present are read later
 #pragma unroll
       for (int e = 0; e < F::V; ++e)
-        W.store(to_f2(x[e]), (rmk[f.l0 + F::first_c(e)] >> r) & 1u ? o.voff(e) : kOff, o.soff(e));
+        W.store(to_f2(x[e]), off_if(rmk[f.l0 + F::first_c(e)], r, o.voff(e)), o.soff(e));
     } else {
 #pragma unroll
       for (int e = 0; e < F::V; ++e) W.store(to_f2(x[e]), o.voff(e), o.soff(e));
