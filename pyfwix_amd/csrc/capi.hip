@@ -380,6 +380,32 @@ KArgs StepEngine::base(int iz, int c0, int np) const {
   return a;
 }
 
+// Planes per launch of a step's passes, at most `chunk` (what the scratch
+// holds).  HBM reads at 4.0 TB/s on this card, the 256 MB memory-side cache at
+// 5.5 and more, writes at 6.9: with several references present per row the per-reference
+// planes W, written by one pass and read by the next, are most of a step's
+// traffic, and a launch whose K and W fit in the cache reads them from there.  The last
+// round of workgroups should still be full, so the planes are a multiple of what
+// fills the chip once (waves a CU holds of the column passes).  11 references (10 present) at 512^2 x 58:
+// 26.3 ms per recursion and adjoint at 58 planes a launch, 26.8 at 15, 22.6 at 12, 23.2 at 10; 4
+// (2.9 present) at 512^2 x 64: 711 us at 64, 648 at 24; 8 at 768^2 x 100: 4.58 ms
+// at 34, 5.3 at 6, 4.42 at 5.  With fewer than 2.5 present per row W is too
+// small a part (FWI at 1024^2, 1.6 present: 48.6 ms at 128, 54.1 at 12).
+static int launch_planes(const fwix_dims& d, int chunk, const std::function<double(int, int)>* rows) {
+  if (!rows) return chunk;
+  const int planes = d.NW * d.NS;
+  const double plane = 8.0 * d.NX * d.NY;
+  if (2.5 * plane * std::min(chunk, planes) < 288e6 / 3) return chunk;  // small: nothing to look up
+  const double live = (*rows)(0, planes) / ((double)planes * d.NY);
+  const int fit = (int)(288e6 / (plane * (1 + live)));
+  if (live < 2.5 || fit >= chunk) return chunk;
+  const bool three = d.NY % 3 == 0;
+  const int waves_per_cu = three ? 16 : d.NY <= 512 ? 24 : 12;
+  const int per_plane = std::max(1, d.NX * (d.NY / (three ? 12 : d.NY <= 512 ? 8 : 16)) / 64);  // column waves
+  const int round = std::max(1, 256 * waves_per_cu / per_plane);
+  return fit < round ? chunk : fit / round * round;
+}
+
 // One depth step over every plane of `in`, run as chunks of `chunk` planes
 // through the three fused passes.  `proto` carries the tables, scratch,
 // depth slices and masks (its p0 / np / wstride are set per chunk);
@@ -395,6 +421,7 @@ void step_passes(int method, bool adjoint, const fwix_dims& d, const fwix_params
   const float sy2 = (float)(1.0 / (double)d.NY);
   const bool pspi = method == FWIX_PSPI;
   const bool taper = pspi && (p.taperx > 0 || p.tapery > 0);
+  chunk = launch_planes(d, chunk, rows);
   for (int c0 = 0; c0 < planes; c0 += chunk) {
     const int np = (planes - c0) < chunk ? (planes - c0) : chunk;
     const double pb = 8.0 * np * plane;  // bytes of one chunk-sized complex64 array
