@@ -209,18 +209,15 @@ struct PlanDef {
 };
 // Row plans and column plans, float32 and float64 arithmetic.
 enum PlanKind { kRow32 = 0, kRow64 = 1, kCol32 = 2, kCol64 = 3 };
-// Rows: short lines take narrow plans (V <= 12): their launches are small and more
-// waves in flight are worth more than a stage less (256 points: Born adjoint
-// rows 21.3 us at V = 16, two stages, 17.5 us at V = 8, three).  The long
-// lines with a factor 3 take V = 24 (768 points: 4 stages of V = 12 against 3);
-// float64 lines hold at most 16 values per lane (twice the registers each).
-// Columns: a first radix R(0) that divides the lanes a wave holds of a column
-// (TileFft), and V <= 12 below 1024 points: these kernels hold two or three
-// arrays of V values per lane (V = 24 at 384 / 768 points, one stage less:
-// fan-out 193 against 180 us / 194 against 198 us, fan-in 233 against 211 us / 262 against
-// 282 us, Taylor-term fan-out 68 against 57 us / 80 against 67 us, 16 M points).
+// Narrow plans (V <= 12 below 1024 points): the kernels hold two or three
+// arrays of V values per lane, short lines' launches are small, and waves in flight
+// are worth more than a stage less (256-point rows: Born adjoint 21.3 us at V = 16,
+// two stages, 17.5 us at V = 8, three; 384 points, V = 24, three stages, against 12, four,
+// 200 planes: scattering adjoint rows 203 -> 151 us, its imaging 129 -> 94, fan-out
+// rows 160 -> 146, fan-out columns 193 -> 180 at 16 M points, fan-in 233 -> 211;
+// 768 points, 5 planes: fan-out rows 52 -> 46 us, the select 39 -> 44).
+// Columns: a first radix R(0) that divides the lanes a wave holds of a column (TileFft).
 __host__ __device__ constexpr PlanDef plan_def(int N, PlanKind kind) {
-  const bool f64 = kind == kRow64 || kind == kCol64, col = kind >= kCol32;
   switch (N) {
     case 8: return {4, 2, {4, 2}};
     case 12: return {12, 1, {12}};
@@ -233,12 +230,12 @@ __host__ __device__ constexpr PlanDef plan_def(int N, PlanKind kind) {
     case 128: return {8, 3, {8, 4, 4}};
     case 192: return {12, 3, {4, 4, 12}};
     case 256: return {8, 3, {8, 8, 4}};
-    case 384: return f64 || col ? PlanDef{12, 4, {4, 4, 4, 6}} : PlanDef{24, 3, {8, 8, 6}};
+    case 384: return {12, 4, {4, 4, 4, 6}};
     case 512: return {8, 3, {8, 8, 8}};
-    case 768: return f64 || col ? PlanDef{12, 4, {4, 4, 4, 12}} : PlanDef{24, 3, {8, 8, 12}};
+    case 768: return {12, 4, {4, 4, 4, 12}};
     case 1024:
       if (kind == kCol64) return {8, 4, {4, 4, 8, 8}};
-      return col ? PlanDef{16, 3, {4, 16, 16}} : PlanDef{16, 3, {16, 8, 8}};
+      return kind == kCol32 ? PlanDef{16, 3, {4, 16, 16}} : PlanDef{16, 3, {16, 8, 8}};
     default: return {0, 0, {}};
   }
 }
