@@ -83,6 +83,14 @@ __device__ __forceinline__ float taylor_coef(int it) {  // Scatter.h:73
   return it == 0 ? 1.f : it == 1 ? 0.5f : it == 2 ? 0.375f : it == 3 ? 0.3125f : 0.2734375f;
 }
 
+// Whether a kernel copies its twiddles to LDS.  These kernels run one or two
+// transforms and have no loop over terms with stores or loads in flight, so
+// at 1024 points their twiddles come from memory (L1): without the 8 KB table a
+// fourth workgroup fits a CU (1024^2 x 128 planes: imaging rows 364 -> 309 us,
+// scattering adjoint rows 800 -> 764).
+template <int N, class T>
+constexpr bool twiddles_in_lds() { return N != 1024 || sizeof(T) == 16; }
+
 // whether any row of this wave lies in the model region (y < ny)
 template <int N, class T>
 __device__ __forceinline__ bool wave_in_model(const KArgs& a, const RowLane<N, T>& w) {
@@ -94,7 +102,8 @@ template <int N, bool MAP>
 __global__ __launch_bounds__(kRowThreads) void k_rows_ic_fwd(KArgs a) {
   using F = LaneFft<N>;
   __shared__ float2 lds[kRowWaves * F::NB * F::STRIDE];
-  __shared__ float2 twl[F::TW];
+  constexpr bool TWL = twiddles_in_lds<N, float2>();
+  __shared__ float2 twl_[TWL ? F::TW : 1];
   const RowLane<N, float2> w(a);
   float2* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   // rows of the padding (y >= ny) carry no product: their spectrum is zero
@@ -111,7 +120,8 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_ic_fwd(KArgs a) {
       return cmul(bg.load_if(i < nx, F::first_c(e)), ds[i < nx ? i : 0]);
     });
   }
-  row_twiddles<N>(twl, a.twx);
+  const float2* twl = TWL ? twl_ : a.twx;
+  if (TWL) row_twiddles<N>(twl_, a.twx);
   __syncthreads();
   if (any) F::template run<false>(v, line, twl, w.l);
   const RowBuf<N, float2> K(a.K, w, a.quad != 0);
@@ -136,7 +146,8 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_scatter(KArgs a) {
   using F = LaneFft<N, T>;
   using S = real_of<T>;
   __shared__ T lds[kRowWaves * F::NB * F::STRIDE];
-  __shared__ T twl[F::TW];
+  constexpr bool TWL = twiddles_in_lds<N, T>();
+  __shared__ T twl_[TWL ? F::TW : 1];
   const RowLane<N, T> w(a);
   T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   const int im = model_iw<MAP>(a, w.iw);
@@ -174,7 +185,8 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_scatter(KArgs a) {
 #pragma unroll
     for (int e = 0; e < F::V; ++e) acc[e] = from_f2<T>(W.load(F::last_c(e)));
   }
-  row_twiddles<N>(twl, twx_of(a, (T*)nullptr));
+  const T* twl = TWL ? twl_ : twx_of(a, (T*)nullptr);
+  if (TWL) row_twiddles<N>(twl_, twx_of(a, (T*)nullptr));
   __syncthreads();
   if (w.empty()) return;
   if constexpr (ONE) {
@@ -238,7 +250,8 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_scatter_adj(KArgs a) {
   using F = LaneFft<N, T>;
   using S = real_of<T>;
   __shared__ T lds[kRowWaves * F::NB * F::STRIDE];
-  __shared__ T twl[F::TW];
+  constexpr bool TWL = twiddles_in_lds<N, T>();
+  __shared__ T twl_[TWL ? F::TW : 1];
   const RowLane<N, T> w(a);
   T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   T u[F::V];
@@ -247,7 +260,8 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_scatter_adj(KArgs a) {
 #pragma unroll
     for (int e = 0; e < F::V; ++e) u[e] = from_f2<T>(in.load(FUSED ? F::last_c(e) : F::first_c(e)));
   }
-  row_twiddles<N>(twl, twx_of(a, (T*)nullptr));
+  const T* twl = TWL ? twl_ : twx_of(a, (T*)nullptr);
+  if (TWL) row_twiddles<N>(twl_, twx_of(a, (T*)nullptr));
   __syncthreads();
   if (w.empty()) return;
   if constexpr (FUSED) {
@@ -313,7 +327,8 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_adj_out(KArgs a) {
   using F = LaneFft<N, T>;
   using S = real_of<T>;
   __shared__ T lds[kRowWaves * F::NB * F::STRIDE];
-  __shared__ T twl[F::TW];
+  constexpr bool TWL = twiddles_in_lds<N, T>();
+  __shared__ T twl_[TWL ? F::TW : 1];
   const RowLane<N, T> w(a);
   T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   // the imaging condition writes the model region only: rows of the
@@ -327,7 +342,8 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_adj_out(KArgs a) {
 #pragma unroll
     for (int e = 0; e < F::V; ++e) x[e] = from_f2<T>(K.load(F::last_c(e)));
   }
-  row_twiddles<N>(twl, twx_of(a, (T*)nullptr));
+  const T* twl = TWL ? twl_ : twx_of(a, (T*)nullptr);
+  if (TWL) row_twiddles<N>(twl_, twx_of(a, (T*)nullptr));
   __syncthreads();
   if (!any) return;
   if (a.nterm > 1) F::template run<true>(x, line, twl, w.l);
