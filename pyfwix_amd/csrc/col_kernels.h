@@ -14,10 +14,10 @@
 // The form before staged every tile through LDS on the way in and out (one
 // exchange and a barrier more per term) and computed every position and LDS address
 // per element.  Before -> now, us per launch: fan-out 512^2 x 64 planes 175 ->
-// 143, 384^2 x 200 375 -> 270, 1024^2 x 128 1012 -> 884, 192 x 384 x 26 (complex
-// slowness) 92 -> 50, 96 x 128 x 24 25 -> 15; fan-in 212 -> 180, 572 -> 335, 1237 -> 1044,
-// 121 -> 53, 25 -> 14; float64 768^2 x 6 fan-out 222 -> 95, fan-in 443 -> 102 (with sincospi and k^2 not held: 134 and
-// 272 before, 117 registers spilled).
+// 143, 384^2 x 200 375 -> 255, 1024^2 x 128 1012 -> 877, 192 x 384 x 26 (complex
+// slowness) 92 -> 50, 96 x 128 x 24 25 -> 11; fan-in 212 -> 180, 572 -> 281, 1237 -> 960,
+// 121 -> 54, 25 -> 10; float64 768^2 x 6 fan-out 222 -> 95, fan-in 443 -> 102 (134 and
+// 272 with sincos and k^2 held, 117 registers spilled).
 #pragma once
 #include "fwix_kernels.h"
 #include "fwix_launch.h"
@@ -144,19 +144,22 @@ __device__ __forceinline__ float2 term_sref(const KArgs& a, int r, int iw) {
 template <int MULT, class T>
 struct TermMult {
   using S = real_of<T>;
-  S w2, wsre, b, iw2, dz;
+  S w2, sre, b, iw2, dz;
+  S turns, decay;  // phase in revolutions and log2 of the amplitude per sqrt|a| (float32, rounded once)
   int r;
   bool real;
   __device__ __forceinline__ TermMult(const KArgs& a, int r_, int iw, S w2_) : w2(w2_), r(r_), dz(a.dz) {
     if constexpr (MULT == 2) {
       iw2 = (S)1 / w2;
-      real = true; wsre = 0; b = 0;
+      real = true; sre = 0; b = 0;
     } else {
       const float2 sr = term_sref(a, r_, iw);
-      wsre = w2 * (S)sr.x;
+      sre = sr.x;
       b = w2 * ((S)sr.y - (S)a.eps * (S)sr.x);
       real = b == 0;
       iw2 = 0;
+      turns = (S)((double)a.dz * 0.15915494309189533577);
+      decay = (S)((double)a.dz * -1.44269504088896340736);
     }
   }
   // x times the multiplier at k2, plus acc where ADD
@@ -181,26 +184,26 @@ struct TermMult {
       return times<ADD>(x, m, acc);
     } else if constexpr (sizeof(S) == 8) {
       if constexpr (!REAL) {
-        return times<ADD>(x, ps_general64<MULT>(wsre - k2, b, dz), acc);
+        return times<ADD>(x, ps_general64<MULT>(w2 * sre - k2, b, dz), acc);
       } else {
-        const S a = wsre - k2, q = sqrt(fabs(a));
+        const S a = w2 * sre - k2, q = sqrt(fabs(a));
         if (a < 0) return times<ADD>(x, exp(-q * dz), acc);
         S sn, cs;
         sincospi(q * (dz * kInvPi), &sn, &cs);
         return times<ADD>(x, CX<T>::mk(cs, MULT == 0 ? -sn : sn), acc);
       }
     } else if constexpr (!REAL) {
-      return times<ADD>(x, ps_general<MULT>(wsre - k2, b, dz), acc);
+      return times<ADD>(x, ps_general<MULT>(fmaf(w2, sre, -k2), b, dz), acc);
     } else {
       // Past the evanescent boundary the multiplier is real and needs no sine
       // or cosine.  A wave's samples are neighbours in (kx, ky), so most
       // waves lie on one side (the propagating disc of a 10-20 m grid covers
       // 3-15 % of the plane): one test of the wave skips both.
-      const float a = wsre - k2, t = __builtin_amdgcn_sqrtf(fabsf(a)) * dz;
-      const float e = __expf(-t);
+      const float a = fmaf(w2, sre, -k2), q = __builtin_amdgcn_sqrtf(fabsf(a));
+      const float e = __builtin_amdgcn_exp2f(q * decay);
       if (__builtin_amdgcn_ballot_w64(a >= 0.f) == 0) return times<ADD>(x, e, acc);
-      float sn, cs;
-      fast_sincos(t, &sn, &cs);
+      const float rev = __builtin_amdgcn_fractf(q * turns);
+      const float sn = __builtin_amdgcn_sinf(rev), cs = __builtin_amdgcn_cosf(rev);
       const float2 m = a >= 0.f ? make_float2(cs, MULT == 0 ? -sn : sn) : make_float2(e, 0.f);
       return times<ADD>(x, m, acc);
     }
