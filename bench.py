@@ -49,6 +49,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import re
 import sys
 import time
 
@@ -63,23 +64,24 @@ COPY_PROBE_TAG = "fwix::k_copy16"   # the probe is the library's 16-byte stream 
                                     # the same kernel and size as the bandwidth probe hbm_copy_gbs
 
 
-def pass_kernel(name, w):
-    """Kernel (demangled name) that a timed pass launches, for the c2-shaped PSPI/Born path
-    (column kernels carry their register budget, row kernels the shot-map flag)."""
+def pass_kernel(name, w, shot_map=False):
+    """Kernel (demangled name) that a timed pass launches in float32 (column kernels carry their register
+    budget and tile width; row kernels whether a shot batch maps planes to shots, and then the select of the
+    chained background steps, which also leaves the next step's spectrum)."""
     from pyfwix_amd import autotune
-    nx, ny = w.NX, w.NY
+    nx, ny, f2, m = w.NX, w.NY, "HIP_vector_type<float, 2u>", str(shot_map).lower()
+
     def col(kind, mode):
         stem, wpe = ("k_cols_fanout", "k_cols_fanin")[kind], autotune.get(kind, mode, ny)
-        if autotune.get_layout(kind, mode, ny) == 1:
-            return f"fwix::{stem}_split<{mode}, {wpe}>"
-        return f"fwix::{stem}<{ny}, {mode}, {wpe}>"
+        cw = 4 if autotune.get_layout(kind, mode, ny) == 1 else 8
+        return f"fwix::{stem}<{ny}, {mode}, {wpe}, {f2}, {cw}" + (", 1>" if kind else ">")
     return {"cols_fanout": col(0, 0), "cols_fanin": col(1, 1),
             "born_cols_kfac": col(0, 2), "born_cols_kfac_adj": col(1, 2),
-            "rows_select": f"fwix::k_rows_select<{nx}, false>", "rows_fanout": f"fwix::k_rows_fanout<{nx}, false>",
-            "born_rows_scatter": f"fwix::k_rows_scatter<{nx}, true, false>",
-            "born_rows_inv_scatter_adj": f"fwix::k_rows_scatter_adj<{nx}, true, false>",
-            "born_rows_adj_ic": f"fwix::k_rows_adj_out<{nx}, true, false>",
-            "born_rows_ic": f"fwix::k_rows_ic_fwd<{nx}, false>"}.get(name)
+            "rows_select": f"fwix::k_rows_select<{nx}, {m}, {m}, 1>", "rows_fanout": f"fwix::k_rows_fanout<{nx}, {m}, {f2} >",
+            "born_rows_scatter": f"fwix::k_rows_scatter<{nx}, true, {m}, {f2}, true>",
+            "born_rows_inv_scatter_adj": f"fwix::k_rows_scatter_adj<{nx}, true, {m}, {f2}, true>",
+            "born_rows_adj_ic": f"fwix::k_rows_adj_out<{nx}, true, {m}, {f2} >",
+            "born_rows_ic": f"fwix::k_rows_ic_fwd<{nx}, {m}>"}.get(name)
 
 
 def _csv_rows(path):
@@ -191,9 +193,10 @@ def _profile_row(path, kernel, ncells, col):
     if kernel in rows:
         return float(rows[kernel].split("/")[0])
     if "k_cols_" in kernel:
-        stem = kernel.rsplit(",", 1)[0]
+        def any_budget(k):
+            return re.sub(r"(<\d+, \d+), \d+", r"\1", k)
         for k, v in rows.items():
-            if k.rsplit(",", 1)[0] == stem:
+            if any_budget(k) == any_budget(kernel):
                 return float(v.split("/")[0])
     return None
 
@@ -803,9 +806,7 @@ def bench_fwi(args):
         NX = NY = N
 
     def kern(name):
-        k = (pass_kernel(name, _W) or "").replace(", false>", ", true>") or None
-        # the background steps are chained: their select pass also leaves the next step's spectrum
-        return f"fwix::k_rows_select<{N}, true, true>" if name == "rows_select" else k
+        return pass_kernel(name, _W, shot_map=True)
     roof = _roofline(passes, args.config, kern, copy_gbs, ev_us)
     lab = N * N * b.planes
     m = nx * nx * b.planes
