@@ -20,10 +20,10 @@ constexpr int kRowThreads = 64 * kRowWaves;
 // has the same winners so far; mode stays in the key.)  The fan-out needs at most
 // 92 registers (113 at 1024 points) and is the same code at every budget but
 // for its schedule (within 3 %).  The fan-in fits 4 waves at V = 8 (16 M points,
-// 512: 223 us at 2, 215 at 4, 275 at 6 with spills); at V = 12 that budget
-// spills (192: 129 / 138 / 129 us, 384: 233 / 244 / 211 us, the third at no
-// budget, which LDS rules out; 768: 315 / 282 / 305 us); at 1024 points LDS holds
-// 3 workgroups and the budgets are equal (210 to 214 us).
+// 512: 235 us at 2, 215 at 4, 210 to 275 at 6, which spills) and, with k^2 formed
+// from LDS, at V = 12, where the budgets are within 4 % (192: 130 / 130 / 129 us,
+// 384: 227 / 219 / 222, 768: 256 / 252 / 249; Taylor terms at 768: 112 / 83 / 112);
+// at 1024 points the budgets are equal (fanin_waves).
 constexpr int col_wpe_default(int kind, int mode, int N) {
   const bool pow2 = !size_has3(N);
   (void)mode;
