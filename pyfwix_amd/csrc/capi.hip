@@ -124,11 +124,16 @@ static std::vector<double2> twiddle_table64(int n) {  // exp(-2 pi i k / n) in d
   }
   return t;
 }
-// the stage twiddles (twiddle_exp) of one kind of plan, in double
-static std::vector<double2> stage_twiddles(int n, PlanKind kind) {
-  const auto t = twiddle_table64(n);
-  std::vector<double2> o(n);
-  for (int i = 0; i < n; ++i) o[i] = t[twiddle_exp(n, kind, i)];
+// the stage twiddles (twiddle_exp, here stage by stage) of one kind of plan
+// from the table t of the length, in double
+static std::vector<double2> stage_twiddles(const std::vector<double2>& t, PlanKind kind) {
+  const int n = (int)t.size();
+  const PlanDef d = plan_def(n, kind);
+  std::vector<double2> o(n, t[0]);
+  int i = 0, ns = d.R[0];
+  for (int s = 1; s < d.S; ns *= d.R[s], ++s)
+    for (int r = 1; r < d.R[s]; ++r)
+      for (int k = 0; k < ns; ++k) o[i++] = t[r * k * (n / (ns * d.R[s]))];
   return o;
 }
 static std::vector<float2> rounded(const std::vector<double2>& t64) {
@@ -177,10 +182,11 @@ void Tables::init(const fwix_dims& d, int tx, int ty) {
   upload_bytes(b_tapx, tx_.data(), tx_.size() * 4);
   upload_bytes(b_tapy, ty_.data(), ty_.size() * 4);
   if (fft_size_supported(d.NX) && fft_size_supported(d.NY)) {
-    auto twx = rounded(stage_twiddles(d.NX, kRow32)), twy = rounded(stage_twiddles(d.NY, kCol32));
+    const auto tx64 = twiddle_table64(d.NX), ty64 = d.NY == d.NX ? tx64 : twiddle_table64(d.NY);
+    auto twx = rounded(stage_twiddles(tx64, kRow32)), twy = rounded(stage_twiddles(ty64, kCol32));
     upload_bytes(b_twx, twx.data(), twx.size() * 8);
     upload_bytes(b_twy, twy.data(), twy.size() * 8);
-    auto twx64 = stage_twiddles(d.NX, kRow64), twy64 = stage_twiddles(d.NY, kCol64);
+    auto twx64 = stage_twiddles(tx64, kRow64), twy64 = stage_twiddles(ty64, kCol64);
     upload_bytes(b_twx64, twx64.data(), twx64.size() * 16);
     upload_bytes(b_twy64, twy64.data(), twy64.size() * 16);
   }
