@@ -141,13 +141,18 @@ struct RowLane {
     iy = row - p * a.NY;
     iw = plane_iw(a, p);
   }
-  __device__ __forceinline__ bool empty() const { return rb >= nrows; }  // wave-uniform
+  // no row at all (wave-uniform): such a wave must not touch memory through a RowBuf
+  __device__ __forceinline__ bool empty() const { return rb >= nrows; }
 };
 // The wave's rows of a wavefield (row-major) or of the K / W scratch (in the
 // launch's layout) as a buffer resource: a lane's elements sit at one 32-bit
 // lane offset plus a uniform offset per element, so they cost no address
 // arithmetic, and the hardware range check reads zero / drops stores of
-// rows beyond the last.
+// rows beyond the last.  The check counts on a wave with at least one row: the
+// lane offset of a row beyond the last is then past the resource whether or not
+// the uniform offset (less than a row, or a quad of rows) is part of it.  A wave
+// without rows has a resource of no bytes based past the array, where a
+// check of lane offset >= size - uniform offset would wrap and let it through.
 template <int N, class T>
 struct RowBuf {
   using F = LaneFft<N, T>;

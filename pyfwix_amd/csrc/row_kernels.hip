@@ -58,6 +58,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows(KArgs a) {
   // K in the quad-block layout goes through LDS as whole lines; row-major K
   // is read and written like any wavefield
   const bool qin = a.qin && a.quad, qout = a.qout && a.quad;
+  if (w.empty() && !qin && !qout) return;  // (the stagings are the whole workgroup's)
   float2* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   const float s = a.scale;  // row normalisation 1/sqrt(NX)
   // positions a transform reads and leaves its values at
@@ -65,13 +66,15 @@ __global__ __launch_bounds__(kRowThreads) void k_rows(KArgs a) {
   auto co = [](int e) { return INV ? F::first_c(e) : F::last_c(e); };
   float2 v[F::V];
   if (!qin) {
-    const RowBuf<N, float2> in(a.in, w, false);
 #pragma unroll
-    for (int e = 0; e < F::V; ++e) v[e] = in.load(ci(e));
+    for (int e = 0; e < F::V; ++e) v[e] = czero();
+    if (!w.empty()) {
+      const RowBuf<N, float2> in(a.in, w, false);
+#pragma unroll
+      for (int e = 0; e < F::V; ++e) v[e] = in.load(ci(e));
+    }
   } else {
     RowStage<N>::load(lds, a.in, R0, w.nrows);
-  }
-  if (qin) {
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < F::V; ++e) v[e] = line[w.l + ci(e)];
@@ -103,6 +106,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows(KArgs a) {
     RowStage<N>::store(lds, a.out, R0, w.nrows);
     return;
   }
+  if (w.empty()) return;
   const RowBuf<N, float2> out(a.out, w, false);
   if (a.add) {
 #pragma unroll
@@ -123,7 +127,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_fanout(KArgs a) {
   T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   T u[F::V];
   Labels<F::V> lab;
-  {
+  if (!w.empty()) {
     const RowBuf<N, T> in(a.in, w, false);
 #pragma unroll
     for (int e = 0; e < F::V; ++e) u[e] = from_f2<T>(in.load(F::first_c(e)));
@@ -185,7 +189,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_select(KArgs a) {
   // this one's transform, except at 16 values per lane or more, where holding
   // it would cost a wave of occupancy
   constexpr bool PREFETCH = F::V < 16;
-  const int rend = a.rowmask ? 32 : a.nref;
+  const int rend = w.empty() ? 0 : a.rowmask ? 32 : a.nref;
   auto after = [&](int r, int k) {  // the k-th reference after r, rend or more when there is none
     for (int i = 0; i < k && r < rend; ++i) r = a.rowmask ? next_bit(live, r) : r + 1;
     return r;
