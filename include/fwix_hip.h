@@ -59,7 +59,7 @@ typedef struct fwix_params {
   float eps;
   float eps_scat;
   int taylor;
-  int planes_per_chunk;     /* planes per fused launch; 0 = automatic */
+  int planes_per_chunk;     /* planes per fused launch, taken as given; 0 = automatic */
 } fwix_params;
 
 /* step methods; FWIX_PSPI_PLAIN runs the PSPI step at the reference's

@@ -387,7 +387,7 @@ KArgs StepEngine::base(int iz, int c0, int np) const {
 }
 
 // Planes per launch of a step's passes, at most `chunk` (what the scratch
-// holds).  HBM reads at 4.0 TB/s on this card, the 256 MB memory-side cache at
+// holds); asked for by step_passes where the caller has not set planes_per_chunk.  HBM reads at 4.0 TB/s on this card, the 256 MB memory-side cache at
 // 5.5 and more, writes at 6.9: with several references present per row the per-reference
 // planes W, written by one pass and read by the next, are most of a step's
 // traffic, and a launch whose K and W fit in the cache reads them from there.  The last
@@ -427,7 +427,7 @@ void step_passes(int method, bool adjoint, const fwix_dims& d, const fwix_params
   const float sy2 = (float)(1.0 / (double)d.NY);
   const bool pspi = method == FWIX_PSPI;
   const bool taper = pspi && (p.taperx > 0 || p.tapery > 0);
-  chunk = launch_planes(d, chunk, rows);
+  if (p.planes_per_chunk == 0) chunk = launch_planes(d, chunk, rows);
   for (int c0 = 0; c0 < planes; c0 += chunk) {
     const int np = (planes - c0) < chunk ? (planes - c0) : chunk;
     const double pb = 8.0 * np * plane;  // bytes of one chunk-sized complex64 array
