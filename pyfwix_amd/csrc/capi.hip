@@ -387,36 +387,61 @@ KArgs StepEngine::base(int iz, int c0, int np) const {
 }
 
 // Planes per launch of a step's passes, at most `chunk` (what the scratch
-// holds); asked for by step_passes where the caller has not set planes_per_chunk.  HBM reads at 4.0 TB/s on this card, the 256 MB memory-side cache at
-// 5.5 and more, writes at 6.9: with several references present per row the per-reference
+// holds); asked for by step_passes where the caller has not set planes_per_chunk.
+// With several references present per row (live, their mean number) the per-reference
 // planes W, written by one pass and read by the next, are most of a step's
-// traffic, and a launch whose K and W fit in the cache reads them from there.  The last
-// round of workgroups should still be full, so the planes are a multiple of what
-// fills the chip once (waves a CU holds of the column passes).  11 references (10 present) at 512^2 x 58:
-// 26.3 ms per recursion and adjoint at 58 planes a launch, 26.8 at 15, 22.6 at 12, 23.2 at 10; 4
-// (2.9 present) at 512^2 x 64: 711 us at 64, 648 at 24; 8 at 768^2 x 100: 4.58 ms
-// at 34, 5.3 at 6, 4.42 at 5.  With fewer than 2.5 present per row W is too
-// small a part (FWI at 1024^2, 1.6 present: 48.6 ms at 128, 54.1 at 12).
-static int launch_planes(const fwix_dims& d, int chunk, const std::function<double(int, int)>* rows) {
-  if (!rows) return chunk;
+// traffic.  HBM reads at 4.0 TB/s on this card, the 256 MB memory-side cache at
+// 5.5 and more, so a launch whose K and W fit in it reads them from there, if
+// it still fills the chip: whole rounds of column workgroups (a round: every
+// CU holds as many as it can) or, where not even one round fits, whole workgroups
+// per CU, at least half of a round (3/4 at 3 2^a points: 384, 16 references, 10 planes a
+// launch 2767 us, all 128 in one 2661).  The launches are then balanced.
+// A PSPI step and its adjoint, random labels (every reference in every row), us
+// with all planes in a launch -> in launches of the planes in brackets:
+//   n x planes    3 references       4                 8                  12
+//   96 x 2048     702 -> 692 (512)   834 -> 790 (512)  1413 -> 1302 (298)  1997 -> 1738 (256)
+//   128 x 1024    637 -> 535 (352)   768 -> 641 (352)  1306 -> 1069 (176)  1826 -> 1489 (128)
+//   192 x 512     708 -> 691 (128)   852 -> 795 (128)  1429 -> 1306 (74)   2001 -> 1807 (64)
+//   256 x 256     627 -> 541 (88)    760 -> 640 (88)   1290 -> 1062 (48)   1801 -> 1524 (32)
+//   384 x 128     739 -> 752 (32)    899 -> 874 (32)   1512 -> 1419 (21)   2095 -> 1971 (16)
+//   512 x 64      637 -> 574 (24)    783 -> 692 (24)   1307 -> 1112 (12)   1837 -> 1528 (8)
+//   768 x 48      whole              whole             2321 -> 2237 (5)    whole
+//   1024 x 32     whole              whole             2775 -> 2562 (3)    3813 -> 3784 (2)
+// (768: in the launches of 24 planes that auto_chunk gives).  Past the size of the cache the gain is
+// gone: 512, 8 references, 60 planes: 988 us at 12 planes a launch, 1065 at 14, 1151 at 16, 1251 at
+// 60.  From 768 points on a launch that fits holds so few planes that it pays only
+// with many references (768, 3: 1113 us at 10 planes, 1088 at 48; 1024, 3: 1331
+// at 6, 1239 at 32; 4: 1618 at 6, 1505; 7: 2272 at 3, 2481).  With two present W is too small
+// a part.  Columns below 96 points have not been measured and stay whole.
+static int launch_planes(const fwix_dims& d, int nref, int chunk, const std::function<double(int, int)>* rows) {
   const int planes = d.NW * d.NS;
-  const double plane = 8.0 * d.NX * d.NY;
-  if (2.5 * plane * std::min(chunk, planes) < 288e6 / 3) return chunk;  // small: nothing to look up
+  const double plane = 8.0 * d.NX * d.NY, cache = 1 << 28;
+  if (!rows || d.NY < 96 || plane * (1 + nref) * std::min(chunk, planes) <= cache) return chunk;
   const double live = (*rows)(0, planes) / ((double)planes * d.NY);
-  const int fit = (int)(288e6 / (plane * (1 + live)));
-  if (live < 2.5 || fit >= chunk) return chunk;
+  if (live < (d.NY < 768 ? 2.5 : 6.5)) return chunk;
+  const int fit = (int)(cache / (plane * (1 + live)));
+  if (fit >= std::min(chunk, planes)) return chunk;
+  // column workgroups: 4 columns at 1024 points, else 8; the waves of one are the
+  // lanes of its columns (V values each), and a CU holds 24, 16 (3 2^a) or 12 (1024) waves
   const bool three = d.NY % 3 == 0;
-  const int waves_per_cu = three ? 16 : d.NY <= 512 ? 24 : 12;
-  const int per_plane = std::max(1, d.NX * (d.NY / (three ? 12 : d.NY <= 512 ? 8 : 16)) / 64);  // column waves
-  const int round = std::max(1, 256 * waves_per_cu / per_plane);
-  return fit < round ? chunk : fit / round * round;
+  const int cw = d.NY == 1024 ? 4 : 8, V = three ? 12 : d.NY == 1024 ? 16 : 8;
+  const int per_cu = (d.NY == 1024 ? 12 : three ? 16 : 24) * 64 / (cw * (d.NY / V));
+  const double one = 256.0 / ((d.NX + cw - 1) / cw);  // planes that put one workgroup on every CU
+  auto planes_of = [&](int k) { return (int)(k * one); };
+  int k = (int)((fit + 1) / one);
+  while (k > 0 && planes_of(k) > fit) --k;
+  if (k >= per_cu) k -= k % per_cu;
+  else if (4 * k < (three ? 3 : 2) * per_cu) return chunk;
+  const int most = planes_of(k), n = (planes + most - 1) / most, share = (planes + n - 1) / n;
+  while (k > 1 && planes_of(k - 1) >= share) --k;
+  return std::max(1, std::min(planes_of(k), chunk));
 }
 
 // One depth step over every plane of `in`, run as chunks of `chunk` planes
 // through the three fused passes.  `proto` carries the tables, scratch,
 // depth slices and masks (its p0 / np / wstride are set per chunk);
 // `rows(p0, np)` gives the per-reference rows a chunk moves, for the pass
-// timers (null: no timers).
+// timers and the size of the launches (null: no timers, launches of `chunk`).
 void step_passes(int method, bool adjoint, const fwix_dims& d, const fwix_params& p, const KArgs& proto, int chunk,
                  int add, const float2* in, float2* out, hipStream_t st,
                  const std::function<double(int, int)>* rows, float2* kall, bool k_ready, bool k_next,
@@ -427,7 +452,7 @@ void step_passes(int method, bool adjoint, const fwix_dims& d, const fwix_params
   const float sy2 = (float)(1.0 / (double)d.NY);
   const bool pspi = method == FWIX_PSPI;
   const bool taper = pspi && (p.taperx > 0 || p.tapery > 0);
-  if (p.planes_per_chunk == 0) chunk = launch_planes(d, chunk, rows);
+  if (p.planes_per_chunk == 0) chunk = launch_planes(d, p.nref, chunk, rows);
   for (int c0 = 0; c0 < planes; c0 += chunk) {
     const int np = (planes - c0) < chunk ? (planes - c0) : chunk;
     const double pb = 8.0 * np * plane;  // bytes of one chunk-sized complex64 array
