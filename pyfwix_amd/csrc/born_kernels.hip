@@ -181,7 +181,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_scatter(KArgs a) {
     return y;
   };
   T acc[F::V];
-  if (ONE && !w.empty()) {
+  if constexpr (ONE) {
     const RowBuf<N, T> W(a.W, w, a.quad != 0);
 #pragma unroll
     for (int e = 0; e < F::V; ++e) acc[e] = from_f2<T>(W.load(F::last_c(e)));
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_scatter_adj(KArgs a) {
   const RowLane<N, T> w(a);
   T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   T u[F::V];
-  if (!w.empty()) {
+  {
     const RowBuf<N, T> in(FUSED ? a.K : a.in, w, FUSED && a.quad != 0);
 #pragma unroll
     for (int e = 0; e < F::V; ++e) u[e] = from_f2<T>(in.load(FUSED ? F::last_c(e) : F::first_c(e)));

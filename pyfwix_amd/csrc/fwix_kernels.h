@@ -141,7 +141,7 @@ struct RowLane {
     iy = row - p * a.NY;
     iw = plane_iw(a, p);
   }
-  // no row at all (wave-uniform): such a wave must not touch memory through a RowBuf
+  // no row at all (wave-uniform): such a wave must not store
   __device__ __forceinline__ bool empty() const { return rb >= nrows; }
 };
 // The wave's rows of a wavefield (row-major) or of the K / W scratch (in the
@@ -151,8 +151,10 @@ struct RowLane {
 // rows beyond the last.  The check counts on a wave with at least one row: the
 // lane offset of a row beyond the last is then past the resource whether or not
 // the uniform offset (less than a row, or a quad of rows) is part of it.  A wave
-// without rows has a resource of no bytes based past the array, where a
-// check of lane offset >= size - uniform offset would wrap and let it through.
+// without rows gets the resource of the first rows, to load from and not to
+// store to: one of no bytes based past the array would let accesses through if
+// the check is lane offset >= size - uniform offset, which wraps.  (No branch
+// around the loads instead: rows_fanout 73.5 against 78.2 us, 768^2 x 24 planes.)
 template <int N, class T>
 struct RowBuf {
   using F = LaneFft<N, T>;
@@ -160,12 +162,12 @@ struct RowBuf {
   unsigned v, row;
   int cs, l;
   __device__ __forceinline__ RowBuf(const float2* base, const RowLane<N, T>& w, bool quad) : l(w.l) {
-    const int r0 = quad ? w.rb & ~3 : w.rb;
+    const int rb = w.empty() ? 0 : w.rb, r0 = quad ? rb & ~3 : rb;
     const int left = w.nrows - r0, most = F::NB + 4;
-    const int rows = left < 0 ? 0 : left < most ? left : most;
+    const int rows = left < most ? left : most;
     r = __builtin_amdgcn_make_buffer_rsrc((void*)(base + (size_t)r0 * N), (short)0,
                                           __builtin_amdgcn_readfirstlane(rows * N * 8), 0x00020000);
-    const unsigned y = (unsigned)(w.rb - r0 + w.b);
+    const unsigned y = (unsigned)(rb - r0 + w.b);
     row = quad ? ((y >> 2) * N + (y & 3)) * 32u : y * N * 8u;
     v = row + (quad ? (((unsigned)l >> 2) << 4) + ((unsigned)l & 3u) : (unsigned)l) * 8u;
     cs = quad ? 32 : 8;

@@ -66,13 +66,9 @@ __global__ __launch_bounds__(kRowThreads) void k_rows(KArgs a) {
   auto co = [](int e) { return INV ? F::first_c(e) : F::last_c(e); };
   float2 v[F::V];
   if (!qin) {
+    const RowBuf<N, float2> in(a.in, w, false);
 #pragma unroll
-    for (int e = 0; e < F::V; ++e) v[e] = czero();
-    if (!w.empty()) {
-      const RowBuf<N, float2> in(a.in, w, false);
-#pragma unroll
-      for (int e = 0; e < F::V; ++e) v[e] = in.load(ci(e));
-    }
+    for (int e = 0; e < F::V; ++e) v[e] = in.load(ci(e));
   } else {
     RowStage<N>::load(lds, a.in, R0, w.nrows);
     __syncthreads();
@@ -127,7 +123,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_fanout(KArgs a) {
   T* line = lds + ((threadIdx.x >> 6) * F::NB + w.b) * F::STRIDE;
   T u[F::V];
   Labels<F::V> lab;
-  if (!w.empty()) {
+  {
     const RowBuf<N, T> in(a.in, w, false);
 #pragma unroll
     for (int e = 0; e < F::V; ++e) u[e] = from_f2<T>(in.load(F::first_c(e)));
