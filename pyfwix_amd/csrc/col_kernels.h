@@ -275,6 +275,10 @@ hipError_t dispatch_mode(int mode, Fn&& fn) {
 // leave the chip idle split their terms (term_split): a fan-out over more
 // workgroups (each with its own forward transform), a fan-in (GROUPS) over thread groups
 // of its workgroups.  K<N, MODE, WPE, T, CW, G>::kernel
+// Tiles of 8 waves (512 and 768 points, 1024 in 8 columns) keep one group: with
+// two of them waiting for each other 4 references take longer on one plane (96 x 512:
+// 16.4 us in two groups, 15.3 in one; 96 x 768: 24.3, 23.9), one present takes 10.9 against
+// 8.9 and 15.3 against 11.9, and 8 gain little (23.5 against 24.2, 36.7 against 39.6).
 constexpr int col_groups(int threads, int N) { return threads <= 128 || N == 256 ? 4 : 2; }
 template <template <int, int, int, class, int, int> class K, bool GROUPS>
 hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) {
@@ -290,7 +294,7 @@ hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) 
         const long long waves = (long long)g.x * g.y * F::WAVES;
         if constexpr (!GROUPS) {
           g.z = term_split(waves, a.nterm, 4, 2048);
-        } else if constexpr (M != 2 && sizeof(T) == 8 && F::THREADS * CW < 4096) {  // (1024 x 8: two regions exceed LDS)
+        } else if constexpr (M != 2 && sizeof(T) == 8 && F::WAVES < 8) {
           constexpr int G = col_groups(F::THREADS, N);
           if (term_split(waves, a.nterm, G, 512) > 1) {
             b.y = G;
