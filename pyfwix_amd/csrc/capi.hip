@@ -348,6 +348,8 @@ void StepEngine::set_refs(const float2* sref_, const uint8_t* labels_) {
             "presence counts");
   present.assign((size_t)nplanes, 0);
   hip_check(hipMemcpy(present.data(), cnt.p, (size_t)nplanes * sizeof(int), hipMemcpyDeviceToHost), "counts D2H");
+  in_plane.assign((size_t)nplanes, 0);
+  hip_check(hipMemcpy(in_plane.data(), planemask.p, (size_t)nplanes * sizeof(uint32_t), hipMemcpyDeviceToHost), "plane masks D2H");
   masks = true;
 }
 
@@ -375,6 +377,9 @@ KArgs StepEngine::base(int iz, int c0, int np) const {
   if (masks) {
     a.rowmask = (const uint32_t*)rowmask.p + (size_t)iz * nmodel * d.NY;
     a.planemask = (const uint32_t*)planemask.p + (size_t)iz * nmodel;
+    const uint32_t refs = params.nref >= 32 ? 0xffffffffu : (1u << params.nref) - 1u;
+    for (int p = 0; p < np; ++p)
+      a.live = std::max(a.live, __builtin_popcount(in_plane[(size_t)iz * nmodel + model_of((c0 + p) % d.NW)] & refs));
   }
   a.nref = params.nref;
   a.nterm = params.nref;

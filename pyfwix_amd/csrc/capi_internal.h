@@ -118,6 +118,7 @@ struct StepEngine {
   DevBuf rowmask, planemask;  // reference presence per (depth, model plane, y) row and per (depth, model plane)
   bool masks = false;
   std::vector<int> present;   // (nz, nmodel): present (row, reference) pairs per model plane
+  std::vector<uint32_t> in_plane;  // (nz, nmodel): planemask on the host
   // Shot batch: plane iw takes its labels / slowness / model from model plane
   // mplane[iw] (the shot it belongs to); nmodel == NW and no map otherwise.
   int nmodel = 0;

@@ -279,6 +279,10 @@ hipError_t dispatch_mode(int mode, Fn&& fn) {
 // two of them waiting for each other 4 references take longer on one plane (96 x 512:
 // 16.4 us in two groups, 15.3 in one; 96 x 768: 24.3, 23.9), one present takes 10.9 against
 // 8.9 and 15.3 against 11.9, and 8 gain little (23.5 against 24.2, 36.7 against 39.6).
+// Groups start at 3 terms (one plane or few, 2 terms, whole -> split: 128 x 128 x 4
+// 8.6 -> 9.3 us, 192 x 192 x 4 10.8 -> 11.7, 384 x 384 13.3 -> 12.9; 3 terms 10.1 -> 9.6, 13.1 ->
+// 12.0, 16.7 -> 16.7), at 256 points at 4 (3: 11.0 -> 11.8; 4: 13.2 -> 12.8, with complex
+// slowness 13.4 -> 13.8; 8: 20.0 -> 18.0).
 constexpr int col_groups(int threads, int N) { return threads <= 128 || N == 256 ? 4 : 2; }
 template <template <int, int, int, class, int, int> class K, bool GROUPS>
 hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) {
@@ -292,11 +296,12 @@ hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) 
         using F = TileFft<N, T, CW>;
         dim3 g = col_grid<F>(a), b(F::THREADS);
         const long long waves = (long long)g.x * g.y * F::WAVES;
+        const int terms = M == 2 ? a.nterm : live_refs(a);
         if constexpr (!GROUPS) {
-          g.z = term_split(waves, a.nterm, 4, 2048);
+          g.z = term_split(waves, terms, 4, 2048);
         } else if constexpr (M != 2 && sizeof(T) == 8 && F::WAVES < 8) {
           constexpr int G = col_groups(F::THREADS, N);
-          if (term_split(waves, a.nterm, G, 512) > 1) {
+          if (term_split(waves, terms, G, 512, N == 256 ? 4 : 3) > 1) {
             b.y = G;
             hipLaunchKernelGGL((K<N, M, 2, T, CW, G>::kernel), g, b, 0, st, a);
             return hipGetLastError();

@@ -62,6 +62,7 @@ struct KArgs {
   float2* aux;             // extra output (checkpoint copy / image)
   int NX, NY, NW, NS, nx, ny;
   int nref, nterm;
+  int live;                // most references present in a plane of the launch (0: unknown)
   int p0, np;              // chunk: first global plane, number of planes
   long long wstride;       // elements between consecutive W terms (np*NX*NY)
   float dz, eps, eps_s;

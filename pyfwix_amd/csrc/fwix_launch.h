@@ -42,12 +42,15 @@ inline long long row_waves(int nrows) {
 // parts meet in LDS it takes less than one: 1024 for the select (192 x 192 x 16,
 // 768 waves: 11.5 -> 10.5 us), 512 for the fan-in, whose groups also wait for each
 // other (192 x 192 x 4, 192 waves: 14.3 -> 12.4 us; x 16, 768 waves: 17.4 -> 22.6).
-inline int term_split(long long waves, int nterm, int most, int limit) {
-  if (waves >= limit || nterm < 2) return 1;
+// nterm counts the references that some plane of the launch holds (KArgs::live):
+// absent ones are skipped and leave parts without work.
+inline int term_split(long long waves, int nterm, int most, int limit, int least = 2) {
+  if (waves >= limit || nterm < least) return 1;
   const long long z = (2048 + waves - 1) / waves;
   const int m = nterm < most ? nterm : most;
   return z < m ? (int)z : m;
 }
+inline int live_refs(const KArgs& a) { return a.live > 0 ? a.live : a.nref; }
 // Argument block of the point-wise operator kernels.
 struct PwArgs {
   int NX, NY, NW, NS;

@@ -321,7 +321,7 @@ hipError_t launch_rows_fanout(const KArgs& a, hipStream_t st) {
     auto go = [&](auto map, auto t) {
       using T = decltype(t);
       dim3 g = row_grid<N, T>(a.np * a.NY);
-      g.y = term_split(row_waves<N, T>(a.np * a.NY), a.nref, 4, 2048);
+      g.y = term_split(row_waves<N, T>(a.np * a.NY), live_refs(a), 4, 2048);
       hipLaunchKernelGGL((k_rows_fanout<N, decltype(map)::value, T>), g, dim3(kRowThreads), 0, st, a);
       return hipGetLastError();
     };
@@ -336,7 +336,7 @@ hipError_t launch_rows_select(const KArgs& a, hipStream_t st) {
     auto go = [&](auto map, auto knext) {
       constexpr bool M = decltype(map)::value, K = decltype(knext)::value;
       const int nrows = a.np * a.NY;
-      const bool split = term_split(row_waves<N, float2>(nrows), a.nref, kRowWaves, 1024) > 1;
+      const bool split = term_split(row_waves<N, float2>(nrows), live_refs(a), kRowWaves, 1024) > 1;
       const dim3 g = row_grid<N, float2>(nrows, split ? kRowWaves : 1);
       if (split) hipLaunchKernelGGL((k_rows_select<N, M, K, kRowWaves>), g, dim3(kRowThreads), 0, st, a);
       else hipLaunchKernelGGL((k_rows_select<N, M, K>), g, dim3(kRowThreads), 0, st, a);
