@@ -354,9 +354,10 @@ int fwix_timing_reset(void);
 int fwix_timing_report(char* buf, int len);
 
 /* ---------------------------------------------------------------- column kernel tuning
- * No counterpart in the reference (cuFFT picks its own kernels).  Every
- * fused column kernel exists with three register budgets: 2, 4 or 6 waves
- * per SIMD.  kind 0 = fan-out transforms (PSPI forward, NSPS adjoint,
+ * No counterpart in the reference (cuFFT picks its own kernels).  The
+ * fused column kernels exist with three register budgets: 2, 4 or 6 waves
+ * per SIMD (where those give the same kernel, it is one: every budget at
+ * n = 1024, 2 and 4 in the fan-in at n = 384).  kind 0 = fan-out transforms (PSPI forward, NSPS adjoint,
  * scattering terms), 1 = fan-in transforms; mode 0 / 1 = forward / adjoint
  * phase shift, 2 = scattering terms; n = column length (NY).
  * fwix_tune_columns_set returns 0, or -1 for an invalid argument;

@@ -1,10 +1,12 @@
 """Autotuner of the fused column kernels.
 
-Every fan-out / fan-in column kernel of the library is compiled for three
+The fan-out / fan-in column kernels of the library are compiled for three
 register budgets, 2, 4 or 6 waves per SIMD (256, 128 or 80 VGPRs).  More
 resident waves hide more of the LDS and HBM latency these transforms wait on,
-but a tight budget can spill, and the workgroup's LDS tile caps residency
+but a tight budget can spill, and the workgroup's LDS caps residency
 anyway; which budget wins depends on the column length and the transform.
+Budgets that would give the same kernel share one (every budget at 1024
+points, 2 and 4 in the fan-in at 384) and one timing.
 :func:`tune_size` times each budget on real launches at one padded grid size
 (a PSPI forward + adjoint step for the phase-shift transforms, modes 0 / 1,
 and a scattering forward + adjoint for the scattering-term transforms, mode
@@ -77,6 +79,13 @@ def load(path: str) -> None:
             set_budget(FANIN, m, int(n), v["fanin"][m])
             set_layout(FANOUT, m, int(n), v.get("fanout_layout", [0, 0, 0])[m])
             set_layout(FANIN, m, int(n), v.get("fanin_layout", [0, 0, 0])[m])
+
+
+def _built(kind: int, n: int, wpe: int) -> int:
+    """Budget of the kernel that a budget selects (``col_wpe_built`` in ``csrc/fwix_kernels.h``)."""
+    if n == 1024:
+        return 2
+    return 4 if kind == FANIN and n == 384 and wpe == 2 else wpe
 
 
 def _time_passes(run, names, reps):
@@ -160,18 +169,25 @@ def tune_size(n: int, planes: int | None = None, nref: int = 4, taylor: int = 1,
         set_budget(k, m, n, lw[1])
 
     out = {"fanout": {}, "fanin": {}, "scatter_fanout": {}, "scatter_fanin": {}}
+    first = {}  # (kind, layout, built budget) -> the first configuration with that kernel
+
+    def record(d, k, lw, t):
+        was = first.setdefault((k, lw[0], _built(k, n, lw[1])), lw)
+        d[key(lw)] = t if was == lw else d[key(was)]
+
     try:
         for lw in configs:
+            kinds = [k for k in (FANOUT, FANIN) if (k, lw[0], _built(k, n, lw[1])) not in first]
             for k in (FANOUT, FANIN):
                 for m in range(3):
                     apply(k, m, lw)
-            t = _time_passes(pspi, ("cols_fanout", "cols_fanin"), reps)
-            out["fanout"][key(lw)] = t.get("cols_fanout")
-            out["fanin"][key(lw)] = t.get("cols_fanin")
+            t = _time_passes(pspi, ("cols_fanout", "cols_fanin"), reps) if kinds else {}
+            record(out["fanout"], FANOUT, lw, t.get("cols_fanout"))
+            record(out["fanin"], FANIN, lw, t.get("cols_fanin"))
             if taylor >= 1:
-                t = _time_passes(scatter, ("scatter_cols", "scatter_cols_adj"), reps)
-                out["scatter_fanout"][key(lw)] = t.get("scatter_cols")
-                out["scatter_fanin"][key(lw)] = t.get("scatter_cols_adj")
+                t = _time_passes(scatter, ("scatter_cols", "scatter_cols_adj"), reps) if kinds else {}
+                record(out["scatter_fanout"], FANOUT, lw, t.get("scatter_cols"))
+                record(out["scatter_fanin"], FANIN, lw, t.get("scatter_cols_adj"))
     except Exception:
         for (k, m), lw in before.items():
             apply(k, m, lw)

@@ -270,7 +270,7 @@ hipError_t dispatch_mode(int mode, Fn&& fn) {
   }
 }
 // One column kernel per (size, mode) and, in float32, register budget (2, 4
-// or 6 waves per SIMD, col_wpe_get) and at 1024 points tile width
+// or 6 waves per SIMD, col_wpe_get, col_wpe_built) and at 1024 points tile width
 // (col_layout_get); float64 arithmetic (a.f64) has one budget.  Launches that
 // leave the chip idle split their terms (term_split): a fan-out over more
 // workgroups (each with its own forward transform), a fan-in (GROUPS) over thread groups
@@ -292,7 +292,7 @@ hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) 
       constexpr int M = decltype(mc)::value;
       auto go = [&](auto wc, auto cc, auto t) -> hipError_t {
         using T = decltype(t);
-        constexpr int CW = decltype(cc)::value, W = decltype(wc)::value;
+        constexpr int CW = decltype(cc)::value, W = col_wpe_built(GROUPS ? 1 : 0, N, decltype(wc)::value);
         using F = TileFft<N, T, CW>;
         dim3 g = col_grid<F>(a), b(F::THREADS);
         const long long waves = (long long)g.x * g.y * F::WAVES;

@@ -8,14 +8,14 @@
 namespace fwix {
 
 // Waves per SIMD the kernel is compiled for under a budget.  LDS admits 3 at
-// 1024 points: 3 (168 registers, 10 spilled) beats 2 for the phase-shift terms (1024^2 x 16
+// 1024 points: 3 (166 registers) beats 2 for the phase-shift terms (1024^2 x 16
 // planes, 202 against 214 us), not for the Taylor terms (75 against 73).  At 384
 // points it admits 4, which the scheduler then has to aim at (219 against 227 us, Taylor terms 70
-// against 78).
+// against 78; col_wpe_built).
 constexpr int fanin_waves(int n, int mode, int wpe, bool f64) {
   if (f64) return 2;
   if (n == 1024) return mode == 2 ? 2 : 3;
-  return n == 384 && wpe < 4 ? 4 : wpe;
+  return wpe;
 }
 
 // (T: arithmetic type of the transforms, float2 or double2; G: groups of

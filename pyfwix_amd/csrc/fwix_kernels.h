@@ -18,17 +18,22 @@ constexpr int kRowThreads = 64 * kRowWaves;
 // launches of every budget on MI355X: kind 0 the fan-out transforms, kind 1
 // the fan-in transforms; mode 2 the scattering terms.  (Every mode of a kind
 // has the same winners so far; mode stays in the key.)  The fan-out needs at most
-// 92 registers (113 at 1024 points) and is the same code at every budget but
+// 93 registers (118 at 1024 points) and is the same code at every budget but
 // for its schedule (within 3 %).  The fan-in fits 4 waves at V = 8 (16 M points,
 // 512: 235 us at 2, 215 at 4, 210 to 275 at 6, which spills) and, with k^2 formed
 // from LDS, at V = 12, where the budgets are within 4 % (192: 130 / 130 / 129 us,
-// 384: 227 / 219 / 222, 768: 256 / 252 / 249; Taylor terms at 768: 112 / 83 / 112);
-// at 1024 points the budgets are equal (fanin_waves).
+// 384: 219 at 2 and 4, 222 at 6, 768: 256 / 252 / 249; Taylor terms at 768: 112 / 83 / 112).
 constexpr int col_wpe_default(int kind, int mode, int N) {
   const bool pow2 = !size_has3(N);
   (void)mode;
   if (kind == 0) return N == 1024 ? 2 : pow2 ? 6 : 4;
   return (pow2 && N <= 512) || N == 768 ? 4 : 2;
+}
+// The budget that a kernel is built for when `wpe` is asked for: where
+// budgets give the same instructions there is one kernel.  At 1024 points that is every budget
+// (LDS decides the waves), in the fan-in at 384 points 2 is 4.
+constexpr int col_wpe_built(int kind, int N, int wpe) {
+  return N == 1024 ? 2 : kind == 1 && N == 384 && wpe == 2 ? 4 : wpe;
 }
 constexpr int kThreads = 256;
 
