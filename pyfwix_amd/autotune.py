@@ -71,14 +71,19 @@ def save(path: str, sizes=(96, 128, 192, 256, 384, 512, 768, 1024)) -> None:
 
 
 def load(path: str) -> None:
+    """Set the table that :func:`save` wrote.  Tune 1024-point columns again where a table holds
+    layout 0 for them and dates from when that was 4 columns with a wave each."""
     with open(path) as f:
         t = json.load(f)
     for n, v in t.items():
         for m in range(3):
             set_budget(FANOUT, m, int(n), v["fanout"][m])
             set_budget(FANIN, m, int(n), v["fanin"][m])
-            set_layout(FANOUT, m, int(n), v.get("fanout_layout", [0, 0, 0])[m])
-            set_layout(FANIN, m, int(n), v.get("fanin_layout", [0, 0, 0])[m])
+            # a table that names no layouts leaves the ones in use
+            if "fanout_layout" in v:
+                set_layout(FANOUT, m, int(n), v["fanout_layout"][m])
+            if "fanin_layout" in v:
+                set_layout(FANIN, m, int(n), v["fanin_layout"][m])
 
 
 def _built(kind: int, n: int, wpe: int) -> int:
