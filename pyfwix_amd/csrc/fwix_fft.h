@@ -216,6 +216,11 @@ enum PlanKind { kRow32 = 0, kRow64 = 1, kCol32 = 2, kCol64 = 3 };
 // 200 planes: scattering adjoint rows 203 -> 151 us, its imaging 129 -> 94, fan-out
 // rows 160 -> 146, fan-out columns 193 -> 180 at 16 M points, fan-in 233 -> 211;
 // 768 points, 5 planes: fan-out rows 52 -> 46 us, the select 39 -> 44).
+// The order of the stages decides whose twiddles' rounding a recursion
+// adds up at its low wavenumbers (the last stage's for the most part): columns of 384 points as
+// {4, 2, 12, 4} take the time of {4, 4, 4, 6} (FWI gradient 384^2 x 200 15.8 ms, steps within
+// 1 %) and leave that gradient 0.93e-6 from float64 instead of 1.27e-6; rows so ordered
+// would halve it again, but read five twiddles more (plain rows 57 -> 62 us, 128 planes).
 // Columns: a first radix R(0) that divides the lanes a wave holds of a column (TileFft).
 __host__ __device__ constexpr PlanDef plan_def(int N, PlanKind kind) {
   switch (N) {
@@ -230,7 +235,7 @@ __host__ __device__ constexpr PlanDef plan_def(int N, PlanKind kind) {
     case 128: return {8, 3, {8, 4, 4}};
     case 192: return {12, 3, {4, 4, 12}};
     case 256: return {8, 3, {8, 8, 4}};
-    case 384: return {12, 4, {4, 4, 4, 6}};
+    case 384: return kind >= kCol32 ? PlanDef{12, 4, {4, 2, 12, 4}} : PlanDef{12, 4, {4, 4, 4, 6}};
     case 512: return {8, 3, {8, 8, 8}};
     case 768: return {12, 4, {4, 4, 4, 12}};
     case 1024:
