@@ -247,21 +247,21 @@ int auto_chunk(const fwix_dims& d, int nterm, int requested) {
   // (row * NX + x), so one chunk stays below 2^31 complex samples.
   const int c_index = (int)std::min<long long>(planes, ((1LL << 31) - 1) / ((long long)d.NX * d.NY));
   if (requested > 0) return std::min(requested, c_index);
-  // Enough planes that a column pass launches >= 32768 workgroups (128 per
-  // CU), so every launch reaches a steady state of loads overlapping
-  // transforms and the partly filled last round of workgroups is a small part
-  // of it.  Born steps (PSPI, 4 references) per padded size, planes per
-  // launch -> Gpts*freq/s: 1024^2 16 -> 32.1, 32 -> 33.8, 128 -> 34.9;
-  // 768^2 43 -> 37.5, 128 -> 39.4, 256 -> 39.8; 512^2 64 -> 55.1, 256 ->
-  // 57.6; 384^2 171 -> 31.0, 256 -> 32.0.  Steps with more than 4 fan-out
-  // planes keep >= 4096 workgroups (16 per CU): NSPS at 768^2 with 8
-  // references, 100 planes, ran 21.25-21.45 at 34 planes per launch and
-  // 20.84-21.31 at 50 or 100.  At most 8 GiB of scratch (spectrum + nterm
-  // fan-out planes).  Chunks are then balanced so the last one is not a
-  // small tail.
+  // Enough planes that a launch holds 128 M points (192 M at 3 2^a points),
+  // counted in blocks of 4096 (6144) of them, at most 32768 planes: it then reaches a
+  // steady state of loads overlapping transforms, and the partly filled last
+  // round of workgroups is a small part of it.  Background, Born forward and adjoint (PSPI, 4
+  // references, smooth model) per padded size, planes per launch -> Gpts*freq/s:
+  // 1024^2 16 -> 39.6, 32 -> 41.9, 64 -> 43.2, 128 -> 43.8; 768^2 43 -> 34.8,
+  // 128 -> 36.9, 256 -> 37.0; 512^2 64 -> 38.4, 128 -> 40.0, 256 -> 41.3; 384^2
+  // 128 -> 35.7, 256 -> 37.2, 512 -> 38.2; 256^2 64 -> 36.7, 256 -> 34.4, 512 ->
+  // 35.9.  Steps with more than 4 fan-out planes hold 16 M (24 M): the scratch they
+  // need per plane is larger, and launch_planes chooses among their launches.
+  // At most 8 GiB of scratch (spectrum + nterm fan-out planes).  Chunks are then
+  // balanced so the last one is not a small tail.
   const double per_plane = (double)(1 + nterm) * d.NX * d.NY * 8.0;
-  const int cw = d.NY >= 1024 ? 4 : d.NY >= 512 ? 8 : std::max(8, (d.NY % 3 == 0 ? 6144 : 4096) / d.NY);
-  const int blocks_per_plane = (d.NX + cw - 1) / cw;
+  const int block = std::max(d.NY % 3 == 0 ? 8 : 4, (d.NY % 3 == 0 ? 6144 : 4096) / d.NY);  // columns of one
+  const int blocks_per_plane = (d.NX + block - 1) / block;
   const int target = nterm > 4 ? 4096 : 32768;
   int c = (target + blocks_per_plane - 1) / blocks_per_plane;
   const int c_max = (int)(8192.0 * 1024 * 1024 / per_plane);

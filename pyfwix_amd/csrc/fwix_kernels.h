@@ -89,19 +89,6 @@ struct KArgs {
 __device__ __forceinline__ unsigned qidx(int y, int x, int NX) {
   return (unsigned)(((((y >> 2) * (NX >> 2)) + (x >> 2)) << 4) + ((y & 3) << 2) + (x & 3));
 }
-// element (y, x) of the K / W scratch in the launch's layout, as a row part
-// (uniform over a row) plus a column part: quad blocks put (y, x) at
-// ((y >> 2) NX + (y & 3)) 4 + ((x >> 2) << 4) + (x & 3)
-__device__ __forceinline__ unsigned wrow(const KArgs& a, int y, int NX) {
-  return a.quad ? (unsigned)(((y >> 2) * NX + (y & 3)) << 2) : (unsigned)(y * NX);
-}
-__device__ __forceinline__ unsigned wcol(const KArgs& a, int x) {
-  const unsigned u = (unsigned)x;
-  return a.quad ? ((u >> 2) << 4) + (u & 3u) : u;
-}
-__device__ __forceinline__ unsigned widx(const KArgs& a, int y, int x, int NX) {
-  return wrow(a, y, NX) + wcol(a, x);
-}
 
 // twiddle tables of the arithmetic type T (float2 or double2)
 __device__ __forceinline__ const float2* twx_of(const KArgs& a, float2*) { return a.twx; }

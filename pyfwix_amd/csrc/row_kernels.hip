@@ -13,7 +13,7 @@
 namespace fwix {
 
 // ------------------------------------------------------------------ row passes
-// A row workgroup covers rows R0 .. R0 + RW NB - 1 (RW = row_waves, R0 a
+// A row workgroup covers rows R0 .. R0 + RW NB - 1 (RW = kRowWaves, R0 a
 // multiple of RW NB), its waves' LDS regions hold those rows in order, STRIDE
 // apart.  In the quad-block layout the same rows are one contiguous run of
 // elements from R0 N, so the workgroup moves them between LDS and memory with
