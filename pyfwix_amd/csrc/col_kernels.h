@@ -17,7 +17,7 @@
 // 143, 384^2 x 200 375 -> 255, 1024^2 x 128 1012 -> 877, 192 x 384 x 26 (complex
 // slowness) 92 -> 50, 96 x 128 x 24 25 -> 11; fan-in 212 -> 180, 572 -> 281, 1237 -> 960,
 // 121 -> 54, 25 -> 10; float64 768^2 x 6 fan-out 222 -> 95, fan-in 443 -> 102 (134 and
-// 272 with sincos and k^2 held, 117 registers spilled).
+// 272 with sincos and k^2 held, 117 registers spilled; 16 now).
 #pragma once
 #include "fwix_kernels.h"
 #include "fwix_launch.h"
@@ -219,10 +219,10 @@ struct TermMult {
 // k^2 = kx^2 + ky^2 at this thread's samples after a forward transform (the
 // positions of the last stage): HELD in registers over the terms, or formed
 // from the wavenumbers staged in LDS (the caller synchronises) where those registers
-// cost waves.  Float64 kernels are at their budget; the float32 fan-in with V = 12 goes
-// from 145 to 126 registers at 384 points, a fourth wave per SIMD, and from 128 with
-// 15 spilled to 126 at 768 (8 references, 34 planes: 543 -> 466 us); with V = 8 the wave
-// more is not reached (512: 215 us held, 222 not).
+// cost waves.  Float64 kernels are at their budget (the phase-shift fan-in with V = 12 still spills 6 to 17
+// of 256); the float32 fan-in with V = 12 goes from 145 to 128 registers at 384 points (3
+// spilled), a fourth wave per SIMD, and from 15 spilled to 2 at 768 (8 references, 34 planes: 543 ->
+// 466 us); with V = 8 the wave more is not reached (512: 215 us held, 222 not).
 template <class F, int N, class S, bool HELD>
 struct ColumnK2 {
   S v[HELD ? F::V : 1];
@@ -299,7 +299,8 @@ hipError_t launch_col_terms(int kind, int mode, const KArgs& a, hipStream_t st) 
       constexpr int M = decltype(mc)::value;
       auto go = [&](auto wc, auto cc, auto t) -> hipError_t {
         using T = decltype(t);
-        constexpr int CW = decltype(cc)::value, W = col_wpe_built(GROUPS ? 1 : 0, N, decltype(wc)::value);
+        constexpr int CW = decltype(cc)::value;
+        constexpr int W = sizeof(T) == 16 ? 2 : col_wpe_built(GROUPS ? 1 : 0, N, decltype(wc)::value);
         using F = TileFft<N, T, CW>;
         dim3 g = col_grid<F>(a), b(F::THREADS);
         const long long waves = (long long)g.x * g.y * F::WAVES;
