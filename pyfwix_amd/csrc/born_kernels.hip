@@ -374,11 +374,13 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_adj_out(KArgs a) {
       if (w.l + F::first_c(e) < nx) aux[w.l + F::first_c(e)] = to_f2(x[e]);
   } else {
     const RowBuf<N, T> out(a.out, w, false);
+    in_groups<F>(x, N, value);  // (loads behind a store to `out` would wait for it: it may be `in`)
+    if (a.add) {
 #pragma unroll
-    for (int e = 0; e < F::V; ++e) {
-      const T y = value(e);
-      out.store(to_f2(a.add ? cadd(from_f2<T>(out.load(F::first_c(e))), y) : y), F::first_c(e));
+      for (int e = 0; e < F::V; ++e) x[e] = cadd(from_f2<T>(out.load(F::first_c(e))), x[e]);
     }
+#pragma unroll
+    for (int e = 0; e < F::V; ++e) out.store(to_f2(x[e]), F::first_c(e));
   }
 }
 
