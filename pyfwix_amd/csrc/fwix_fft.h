@@ -222,6 +222,10 @@ enum PlanKind { kRow32 = 0, kRow64 = 1, kCol32 = 2, kCol64 = 3 };
 // 200 planes: scattering adjoint rows 203 -> 151 us, its imaging 129 -> 94, fan-out
 // rows 160 -> 146, fan-out columns 193 -> 180 at 16 M points, fan-in 233 -> 211;
 // 768 points, 5 planes: fan-out rows 52 -> 46 us, the select 39 -> 44).
+// Rows of 12 and 24 points hold 6 values per lane, two and four lanes to a row: with 12, one and
+// two lanes, an access touches 64 or 32 rows (12 x 1024 x 341 planes: plain rows 26 -> 17 us,
+// scattering rows 48 -> 28, imaging rows 47 -> 27; 24 x 768 x 227: 18 -> 14, 31 -> 22, 32 -> 21).
+// Columns lie across a tile and keep 12.
 // The order of the stages decides whose twiddles' rounding a recursion
 // adds up at its low wavenumbers (the last stage's for the most part): columns of 384 points as
 // {4, 2, 12, 4} take the time of {4, 4, 4, 6} (FWI gradient 384^2 x 200 15.8 ms, steps within
@@ -231,9 +235,9 @@ enum PlanKind { kRow32 = 0, kRow64 = 1, kCol32 = 2, kCol64 = 3 };
 __host__ __device__ constexpr PlanDef plan_def(int N, PlanKind kind) {
   switch (N) {
     case 8: return {4, 2, {4, 2}};
-    case 12: return {12, 1, {12}};
+    case 12: return kind >= kCol32 ? PlanDef{12, 1, {12}} : PlanDef{6, 2, {6, 2}};
     case 16: return {4, 2, {4, 4}};
-    case 24: return {12, 2, {4, 6}};
+    case 24: return kind >= kCol32 ? PlanDef{12, 2, {4, 6}} : PlanDef{6, 3, {2, 6, 2}};
     case 32: return {8, 2, {8, 4}};
     case 48: return {12, 2, {4, 12}};
     case 64: return {8, 2, {8, 8}};
