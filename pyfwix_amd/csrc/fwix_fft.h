@@ -226,8 +226,8 @@ enum PlanKind { kRow32 = 0, kRow64 = 1, kCol32 = 2, kCol64 = 3 };
 // two lanes, an access touches 64 or 32 rows (12 x 1024 x 341 planes: plain rows 26 -> 17 us,
 // scattering rows 48 -> 28, imaging rows 47 -> 27; 24 x 768 x 227: 18 -> 14, 31 -> 22, 32 -> 21).
 // Columns lie across a tile and keep 12.
-// The order of the stages decides whose twiddles' rounding a recursion
-// adds up at its low wavenumbers (the last stage's for the most part): columns of 384 points as
+// The order of the stages decides which twiddles' rounding a recursion
+// adds up step after step: columns of 384 points as
 // {4, 2, 12, 4} take the time of {4, 4, 4, 6} (FWI gradient 384^2 x 200 15.8 ms, steps within
 // 1 %) and leave that gradient 0.93e-6 from float64 instead of 1.27e-6; rows so ordered
 // would halve it again, but read five twiddles more (plain rows 57 -> 62 us, 128 planes).
